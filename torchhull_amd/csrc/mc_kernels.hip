@@ -528,8 +528,9 @@ mc_edge_vertices(const McPlan& p, const Lookup& lk, const McGrid& g, uint64_t i,
 // processed with all lanes busy.  The outputs of a batch of queued vertices are still one
 // contiguous range (the vertices between them emit nothing), assembled in LDS and written with
 // coalesced stores.
-// 64-vertex chunks per wavefront (measured on the mixed workload: 16 and 32 chunks, 148 vs 153 and
-// 182 us for the vertices; 8, 16 and 32 chunks, 283, 278 and 308 us for the faces)
+// 64-vertex chunks per wavefront: at most kMcVertexChunks and kMcFaceChunks (measured on the mixed
+// workload: 16 and 32 chunks, 148 vs 153 and 182 us for the vertices; 8, 16 and 32 chunks, 283, 278 and
+// 308 us for the faces), fewer for lists that would leave CUs idle (mc_chunks).
 constexpr int kMcVertexChunks = 8;
 constexpr int kMcFaceChunks = 16;
 
@@ -602,15 +603,15 @@ mc_vertices_batch(const McPlan& p, const Lookup& lk, const McQueue& Q, uint32_t 
 
 template <typename Lookup, typename V>
 __global__ __launch_bounds__(256) void
-mc_vertices_kernel(McPlan p, Lookup lk, const uint32_t* __restrict__ emask, const uint32_t* __restrict__ vbase,
-                   float* __restrict__ verts)
+mc_vertices_kernel(McPlan p, Lookup lk, int chunks, const uint32_t* __restrict__ emask,
+                   const uint32_t* __restrict__ vbase, float* __restrict__ verts)
 {
     __shared__ float stage[kMcWaves][64 * 3 * 3];
     __shared__ McQueue queue[kMcWaves];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint64_t v0 = (uint64_t(xcd_block(blockIdx.x, gridDim.x)) * kMcWaves + wave) * (64u * kMcVertexChunks);
+    const uint64_t v0 = (uint64_t(xcd_block(blockIdx.x, gridDim.x)) * kMcWaves + wave) * (64u * uint32_t(chunks));
     uint32_t q = 0u; // queued vertices (wave-uniform)
-    for (int c = 0; c < kMcVertexChunks; ++c)
+    for (int c = 0; c < chunks; ++c)
     {
         const uint64_t i = v0 + 64u * uint32_t(c) + lane;
         if (v0 + 64u * uint32_t(c) >= p.nverts)
@@ -856,6 +857,7 @@ template <typename Lookup>
 __global__ __launch_bounds__(256) void
 mc_faces_unique_kernel(McPlan p,
                        Lookup lk,
+                       int chunks,
                        const uint32_t* __restrict__ info,
                        const uint32_t* __restrict__ tbase,
                        const uint32_t* __restrict__ emask,
@@ -866,9 +868,9 @@ mc_faces_unique_kernel(McPlan p,
     __shared__ uint32_t stage[kMcWaves][64 * kMcMaxTriVerts];
     __shared__ McQueue queue[kMcWaves];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint64_t v0 = (uint64_t(xcd_block(blockIdx.x, gridDim.x)) * kMcWaves + wave) * (64u * kMcFaceChunks);
+    const uint64_t v0 = (uint64_t(xcd_block(blockIdx.x, gridDim.x)) * kMcWaves + wave) * (64u * uint32_t(chunks));
     uint32_t q = 0u; // queued cells (wave-uniform)
-    for (int c = 0; c < kMcFaceChunks; ++c)
+    for (int c = 0; c < chunks; ++c)
     {
         const uint64_t i = v0 + 64u * uint32_t(c) + lane;
         if (v0 + 64u * uint32_t(c) >= p.nverts)
@@ -894,6 +896,18 @@ mc_faces_unique_kernel(McPlan p,
 // ---------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------
+
+// Chunks per wavefront of the gathering kernels: `most` where that still gives kMcTargetWaves wavefronts
+// (16 per CU), else as many as give them, since a wavefront walks its chunks one after the other and each
+// batch is a chain of dependent reads.  Level-7 hull of 8 cameras (about 60 000 vertices): faces 42 -> 7.7 us
+// and vertices 16 -> 4.9 us; sparse 400^3 sphere band (1.5 million): faces 51 -> 29 us.
+constexpr uint64_t kMcTargetWaves = 4096;
+
+static int
+mc_chunks(uint64_t nverts, int most)
+{
+    return int(std::min<uint64_t>(uint64_t(most), std::max<uint64_t>(1, nverts / (64u * kMcTargetWaves))));
+}
 
 // Workgroups of the gathering kernels: kMcWaves wavefronts of `chunks` 64-vertex chunks each.
 static unsigned
@@ -958,7 +972,9 @@ launch_mc_vertices(const McPlan& p, const uint32_t* emask, const uint32_t* vbase
     dispatch_mc(p, [&](auto lk, auto vt) {
         using LK = decltype(lk);
         using VT = decltype(vt);
-        mc_vertices_kernel<LK, VT><<<mc_gather_blocks(p.nverts, kMcVertexChunks), 256, 0, st>>>(p, lk, emask, vbase, verts);
+        const int chunks = mc_chunks(p.nverts, kMcVertexChunks);
+        mc_vertices_kernel<LK, VT><<<mc_gather_blocks(p.nverts, chunks), 256, 0, st>>>(p, lk, chunks, emask, vbase,
+                                                                                      verts);
     });
     THULL_LAUNCH_CHECK();
 }
@@ -981,9 +997,10 @@ launch_mc_faces(const McPlan& p,
     dispatch_mc(p, [&](auto lk, auto vt) {
         using LK = decltype(lk);
         using VT = decltype(vt);
+        const int chunks = mc_chunks(p.nverts, kMcFaceChunks);
         if (unique)
-            mc_faces_unique_kernel<LK><<<mc_gather_blocks(p.nverts, kMcFaceChunks), 256, 0, st>>>(
-                    p, lk, info, ntv_base, emask, vbase, scene_vstart, faces);
+            mc_faces_unique_kernel<LK><<<mc_gather_blocks(p.nverts, chunks), 256, 0, st>>>(
+                    p, lk, chunks, info, ntv_base, emask, vbase, scene_vstart, faces);
         else
             mc_faces_kernel<LK, VT><<<blocks_for(int64_t(p.nverts), 256), 256, 0, st>>>(
                     p, lk, info, ntv_base, emask, vbase, scene_vstart, scene_tstart, unique, soup_verts, faces);
