@@ -1132,7 +1132,6 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
     plan.iso = 0.5f;
     plan.bitmap = bitmap;
     plan.prefix = prefix;
-    plan.dense = false;
 
     uint64_t vtotal = 0, ttotal = 0;
     float* verts = nullptr;
@@ -1679,18 +1678,52 @@ thull_marching_cubes_dense_run(thull_ctx* ctx,
         Context& c = ctx->c;
         hipStream_t st = static_cast<hipStream_t>(stream);
         c.begin(st);
-        McPlan plan{};
-        plan.vertices = nullptr;
-        plan.nverts = (D < 2 || H < 2 || W < 2) ? 0 : uint64_t(D * H * W);
-        plan.values = volume;
-        plan.value_type = dtype == kF64 ? kMcF64 : kMcF32;
-        plan.iso = isolevel;
-        plan.dense = true;
-        plan.dense_dims[0] = uint32_t(W);
-        plan.dense_dims[1] = uint32_t(H);
-        plan.dense_dims[2] = uint32_t(D);
-        mc_run_common(c, plan, upload_mc_grid(c, mc_grid(D, H, W, return_local_coords != 0), st), unique_verts != 0,
-                      st, num_verts, num_faces);
+        Pool& pool = c.pool;
+        *num_verts = *num_faces = 0;
+        if (D < 2 || H < 2 || W < 2)
+        {
+            c.mc_valid = true;
+            return;
+        }
+        McDense d{};
+        d.dims[0] = uint32_t(W);
+        d.dims[1] = uint32_t(H);
+        d.dims[2] = uint32_t(D);
+        d.row_words = uint32_t((W + 31) / 32);
+        d.nwords = uint64_t(d.row_words) * uint64_t(H) * uint64_t(D);
+        d.signs = pool.alloc<uint32_t>(d.nwords);
+        const int32_t value_type = dtype == kF64 ? kMcF64 : kMcF32;
+        const uint32_t tiles = mc_dense_tiles(d.nwords);
+        void* edges = pool.alloc_bytes(mc_dense_edge_bytes(d.nwords));
+        uint32_t* counts = pool.alloc<uint32_t>(d.nwords);
+        uint32_t* tile_verts = pool.alloc<uint32_t>(uint64_t(tiles) + 3); // scanned in groups of 4
+        uint32_t* tile_tris = pool.alloc<uint32_t>(uint64_t(tiles) + 3);
+        unsigned long long* totals = pool.alloc<unsigned long long>(2); // output vertices, triangle vertices
+        launch_mc_dense_counts(d, volume, value_type, isolevel, edges, counts, tile_verts, tile_tris, st);
+        const ScanNotify note = c.notify.next(nullptr);
+        scan_block_sums2_kernel<><<<1, 1024, 0, st>>>(tile_verts, tile_tris, tiles, totals, note);
+        THULL_LAUNCH_CHECK();
+        unsigned long long got[2];
+        if (!c.notify.wait(note, st, got))
+        {
+            THULL_HIP(hipMemcpyAsync(c.stage->p, totals, sizeof(got), hipMemcpyDeviceToHost, st));
+            THULL_HIP(hipStreamSynchronize(st));
+            got[0] = c.stage->p[0];
+            got[1] = c.stage->p[1];
+        }
+        const bool unique = unique_verts != 0;
+        const uint64_t ttotal = got[1], vtotal = unique ? got[0] : ttotal;
+        check_u32(ttotal, "triangle vertex count");
+        c.mc_verts = pool.alloc<float>(3 * std::max<uint64_t>(vtotal, 1));
+        c.mc_faces = pool.alloc<int64_t>(std::max<uint64_t>(ttotal, 1));
+        if (ttotal > 0)
+            launch_mc_dense_mesh(d, mc_grid(D, H, W, return_local_coords != 0), volume, value_type, isolevel, counts,
+                                 tile_verts, tile_tris, edges, unique, c.mc_verts, c.mc_faces, st);
+        c.mc_nv = int64_t(vtotal);
+        c.mc_nf = int64_t(ttotal / 3);
+        *num_verts = c.mc_nv;
+        *num_faces = c.mc_nf;
+        c.mc_valid = true;
     });
 }
 
@@ -1761,7 +1794,6 @@ thull_marching_cubes_sparse_run(thull_ctx* ctx,
         plan.values = values;
         plan.value_type = dtype == kF64 ? kMcF64 : kMcF32;
         plan.iso = isolevel;
-        plan.dense = false;
         mc_run_common(c, plan, up, unique_verts != 0, st, num_verts, num_faces);
     });
 }

@@ -93,9 +93,7 @@ void launch_wireframe(const int64_t* cells, uint32_t n, int32_t level, const flo
 
 // ---- marching cubes (mc_kernels.hip) ----
 
-// Grid description for marching cubes.  For the bitmap policy, vertex
-// positions are ranks in the batch bitmap; for the dense policy the vertex of
-// (x, y, z) is at x + dims[0] * (y + dims[1] * z).
+// Grid description for marching cubes.  Vertex positions of the sparse passes are ranks in the batch bitmap.
 struct McGrid
 {
     uint32_t dims[3];       // grid vertices per axis
@@ -117,15 +115,13 @@ struct McPlan
 {
     // inputs
     const McGrid* grids;      // device, one per scene
-    const uint64_t* vertices; // packed keys (bitmap policy); null for the dense policy
-    uint64_t nverts;          // vertex count (dense: dims product)
+    const uint64_t* vertices; // packed keys
+    uint64_t nverts;          // vertex count
     const void* values;       // [nverts] f32 or f64
     int32_t value_type;
     float iso;
-    const uint32_t* bitmap;   // bitmap policy
-    const uint32_t* prefix;   // bitmap policy: exclusive popcount prefix per word
-    bool dense;
-    uint32_t dense_dims[3];
+    const uint32_t* bitmap;   // grid vertices
+    const uint32_t* prefix;   // exclusive popcount prefix per word
 };
 
 // Pass 1: per vertex info word (case, complete bit, edge sign-change bits) and
@@ -141,6 +137,25 @@ void launch_mc_vertices(const McPlan& p, const uint32_t* emask, const uint32_t* 
 void launch_mc_faces(const McPlan& p, const uint32_t* info, const uint32_t* ntv_base, const uint32_t* emask,
                      const uint32_t* vbase, const uint32_t* scene_vstart, const uint32_t* scene_tstart, bool unique,
                      float* soup_verts, int64_t* faces, hipStream_t st);
+
+// Dense volumes [D,H,W] (x fastest) of at least 2 points per axis and fewer than 2^32 points.
+struct McDense
+{
+    uint32_t dims[3];   // points along x, y, z
+    uint32_t row_words; // 32-point words per row
+    uint64_t nwords;    // row_words * dims[1] * dims[2]
+    uint32_t* signs;    // [nwords] one bit per point: value below the isolevel
+};
+uint32_t mc_dense_tiles(uint64_t nwords);
+size_t mc_dense_edge_bytes(uint64_t nwords);
+// Sign bits, edge masks (`edges`, mc_dense_edge_bytes) and counts of every word ([nwords]), and the counts of
+// output vertices and triangle vertices of every tile (mc_dense_tiles entries each).
+void launch_mc_dense_counts(const McDense& d, const void* volume, int32_t value_type, float iso, void* edges,
+                            uint32_t* counts, uint32_t* tile_verts, uint32_t* tile_tris, hipStream_t st);
+// The mesh, from the exclusive prefixes of the tile counts; soups (unique false) have a vertex per triangle corner.
+void launch_mc_dense_mesh(const McDense& d, const McGrid& g, const void* volume, int32_t value_type, float iso,
+                          const uint32_t* counts, const uint32_t* tile_verts, const uint32_t* tile_tris, void* edges,
+                          bool unique, float* verts, int64_t* faces, hipStream_t st);
 
 // Grid-vertex bitmap of a sparse COO volume: marks (x, y, z) = (idx[3], idx[2], idx[1]).  An entry outside the
 // volume (or with a negative index idx[0]) marks nothing and sets *bad.

@@ -24,6 +24,7 @@
 
 #include "mc_cases.h"
 #include "kernels.h"
+#include "scan.h"
 
 namespace thull
 {
@@ -88,36 +89,6 @@ struct BitmapLookup
     }
 };
 
-struct DenseLookup
-{
-    __device__ __forceinline__ bool
-    find(const McGrid& g, uint32_t x, uint32_t y, uint32_t z, uint32_t& pos) const
-    {
-        pos = x + g.dims[0] * (y + g.dims[1] * z);
-        return true;
-    }
-
-    struct Probe
-    {
-        uint32_t pos;
-    };
-    __device__ __forceinline__ Probe
-    probe(const McGrid& g, uint32_t x, uint32_t y, uint32_t z) const
-    {
-        return Probe{ x + g.dims[0] * (y + g.dims[1] * z) };
-    }
-    __device__ __forceinline__ bool
-    present(const Probe&) const
-    {
-        return true;
-    }
-    __device__ __forceinline__ uint32_t
-    rank(const Probe& p) const
-    {
-        return p.pos;
-    }
-};
-
 struct VertexRef
 {
     uint32_t scene, x, y, z;
@@ -126,13 +97,6 @@ struct VertexRef
 __device__ __forceinline__ VertexRef
 vertex_ref(const McPlan& p, uint64_t i)
 {
-    if (p.dense)
-    {
-        const uint64_t sx = p.dense_dims[0], sy = p.dense_dims[1];
-        const uint64_t row = div_u64_u32(i, uint32_t(sx));
-        const uint64_t z = div_u64_u32(row, uint32_t(sy));
-        return VertexRef{ 0u, uint32_t(i - row * sx), uint32_t(row - z * sy), uint32_t(z) };
-    }
     const uint64_t k = p.vertices[i];
     return VertexRef{ key_scene(k), key_x(k), key_y(k), key_z(k) };
 }
@@ -200,34 +164,9 @@ finish_vertex(const McGrid& g, const float v[3], float* out)
 // Pass 1: cell case, completeness and edge sign changes per vertex
 // ---------------------------------------------------------------------------
 
-// Presence and rank of the cell's 7 other corners, in case-corner order 1, 4,
-// 3 (the +x, +y, +z neighbours), then 2, 5, 6, 7.  found[k]: inside the grid
-// and present; pos[k] is set where `need` says so (rank reads only for those).
-// With the bitmap policy the two corners x and x + 1 of one (y, z) row share a
-// bitmap word (and its prefix): 3 row words plus the vertex's own word are
-// read instead of 7 words and 7 prefixes, and the +x neighbour of a present
-// vertex i is vertex i + 1.
-template <typename Lookup>
-__device__ __forceinline__ void
-cell_corners(const Lookup& lk, const McGrid& g, uint64_t i, const VertexRef& r, bool (&found)[7],
-             typename Lookup::Probe (&pr)[7], bool& inx, bool& iny, bool& inz)
-{
-    constexpr uint32_t corner[7] = { 1u, 4u, 3u, 2u, 5u, 6u, 7u };
-    inx = r.x + 1 < g.dims[0];
-    iny = r.y + 1 < g.dims[1];
-    inz = r.z + 1 < g.dims[2];
-#pragma unroll
-    for (int k = 0; k < 7; ++k)
-    {
-        const uint32_t o = c_corner_off_host[corner[k]];
-        const bool in = (!(o & 1u) || inx) && (!((o >> 1) & 1u) || iny) && (!((o >> 2) & 1u) || inz);
-        if (in)
-            pr[k] = lk.probe(g, r.x + (o & 1u), r.y + ((o >> 1) & 1u), r.z + ((o >> 2) & 1u));
-        found[k] = in && lk.present(pr[k]);
-    }
-}
-
-// Bitmap policy: row words shared by the corners x and x + 1.
+// The two corners x and x + 1 of one (y, z) row of a cell share a bitmap word (and its prefix): 3 row
+// words plus the vertex's own word are read instead of 7 words and 7 prefixes, and the +x neighbour of a
+// present vertex i is vertex i + 1.
 struct RowProbe
 {
     uint64_t w;     // word of x
@@ -256,135 +195,97 @@ row_probe(const BitmapLookup& lk, const McGrid& g, uint32_t x, uint32_t y, uint3
     return q;
 }
 
-template <typename Lookup, typename V, bool UNIFORM>
+template <typename V, bool UNIFORM>
 __device__ __forceinline__ void
-mc_classify_vertex(const McPlan& p, const Lookup& lk, const McGrid& g, uint64_t i, const VertexRef& r, uint32_t& info,
-                   uint32_t& ntv)
+mc_classify_vertex(const McPlan& p, const BitmapLookup& lk, const McGrid& g, uint64_t i, const VertexRef& r,
+                   uint32_t& info, uint32_t& ntv)
 {
     const V iso = static_cast<V>(p.iso);
     constexpr uint32_t corner[7] = { 1u, 4u, 3u, 2u, 5u, 6u, 7u };
     bool found[7];
-    uint32_t pos[7];
     bool inx, iny, inz;
-    if constexpr (std::is_same_v<Lookup, BitmapLookup>)
+    inx = r.x + 1 < g.dims[0];
+    iny = r.y + 1 < g.dims[1];
+    inz = r.z + 1 < g.dims[2];
+    // rows (dy, dz) = (0, 0), (1, 0), (0, 1), (1, 1); row (0, 0) holds the vertex itself
+    const RowProbe q00 = row_probe(lk, g, r.x, r.y, r.z, true, inx);
+    const RowProbe q10 = row_probe(lk, g, r.x, r.y + 1, r.z, iny, inx);
+    const RowProbe q01 = row_probe(lk, g, r.x, r.y, r.z + 1, inz, inx);
+    const RowProbe q11 = row_probe(lk, g, r.x, r.y + 1, r.z + 1, iny && inz, inx);
+    // corners 1 (x+1,y,z), 4 (x,y+1,z), 3 (x,y,z+1), 2 (x+1,y,z+1), 5 (x+1,y+1,z), 6 (x+1,y+1,z+1), 7 (x,y+1,z+1)
+    found[0] = q00.p1;
+    found[1] = q10.p0;
+    found[2] = q01.p0;
+    found[3] = q01.p1;
+    found[4] = q10.p1;
+    found[5] = q11.p1;
+    found[6] = q11.p0;
+    bool complete = inx && iny && inz; // MC:199
+#pragma unroll
+    for (int k = 0; k < 7; ++k)
+        complete = complete && found[k];
+    // Values are read as pairs of consecutive vertices, the corners x and x + 1 of a row: the
+    // vertex itself and its +x neighbour (which follows it when present), and in the rows
+    // (y + 1, z), (y, z + 1), (y + 1, z + 1) the first present corner x' at rank r of x and, in a
+    // complete cell, x + 1 at r + 1.  A pair starts at a = min(r, nverts - 2) (some neighbour is
+    // present whenever one is read, so nverts >= 2), and the value of r is its first element when
+    // a == r, else its second (r = nverts - 1); the second corner of a pair is only read in a
+    // complete cell, where r + 1 < nverts.
+    typedef V pair_t __attribute__((ext_vector_type(2), aligned(sizeof(V))));
+    typedef __attribute__((address_space(1))) const pair_t global_pair_t;
+    const V* vals = static_cast<const V*>(p.values);
+    const uint32_t last2 = uint32_t(p.nverts) - 2u; // used only when nverts >= 2
+    V vg, vrow[4][2] = {}; // entries of absent corners are never compared
+    if (found[0])
     {
-        inx = r.x + 1 < g.dims[0];
-        iny = r.y + 1 < g.dims[1];
-        inz = r.z + 1 < g.dims[2];
-        // rows (dy, dz) = (0, 0), (1, 0), (0, 1), (1, 1); row (0, 0) holds the vertex itself
-        const RowProbe q00 = row_probe(lk, g, r.x, r.y, r.z, true, inx);
-        const RowProbe q10 = row_probe(lk, g, r.x, r.y + 1, r.z, iny, inx);
-        const RowProbe q01 = row_probe(lk, g, r.x, r.y, r.z + 1, inz, inx);
-        const RowProbe q11 = row_probe(lk, g, r.x, r.y + 1, r.z + 1, iny && inz, inx);
-        // corners 1 (x+1,y,z), 4 (x,y+1,z), 3 (x,y,z+1), 2 (x+1,y,z+1), 5 (x+1,y+1,z), 6 (x+1,y+1,z+1), 7 (x,y+1,z+1)
-        found[0] = q00.p1;
-        found[1] = q10.p0;
-        found[2] = q01.p0;
-        found[3] = q01.p1;
-        found[4] = q10.p1;
-        found[5] = q11.p1;
-        found[6] = q11.p0;
-        bool complete = inx && iny && inz; // MC:199
-#pragma unroll
-        for (int k = 0; k < 7; ++k)
-            complete = complete && found[k];
-        // Values are read as pairs of consecutive vertices, the corners x and x + 1 of a row: the
-        // vertex itself and its +x neighbour (which follows it when present), and in the rows
-        // (y + 1, z), (y, z + 1), (y + 1, z + 1) the first present corner x' at rank r of x and, in a
-        // complete cell, x + 1 at r + 1.  A pair starts at a = min(r, nverts - 2) (some neighbour is
-        // present whenever one is read, so nverts >= 2), and the value of r is its first element when
-        // a == r, else its second (r = nverts - 1); the second corner of a pair is only read in a
-        // complete cell, where r + 1 < nverts.
-        typedef V pair_t __attribute__((ext_vector_type(2), aligned(sizeof(V))));
-        typedef __attribute__((address_space(1))) const pair_t global_pair_t;
-        const V* vals = static_cast<const V*>(p.values);
-        const uint32_t last2 = uint32_t(p.nverts) - 2u; // used only when nverts >= 2
-        V vg, vrow[4][2] = {}; // entries of absent corners are never compared
-        if (found[0])
-        {
-            const pair_t v2 = *(global_pair_t*)(vals + i); // i + 1 < nverts
-            vg = v2.x;
-            vrow[0][1] = v2.y;
-        }
-        else
-            vg = vals[i];
-        const auto row_pair = [&](const RowProbe& q, int row) {
-            const uint32_t b = r.x & 31u;
-            const uint32_t r0 = q.pre + __popc(q.word & ((1u << b) - 1u));
-            const uint32_t a = min(r0, last2);
-            const pair_t v2 = *(global_pair_t*)(vals + a);
-            vrow[row][0] = a == r0 ? v2.x : v2.y;
-            vrow[row][1] = v2.y;
-        };
-        if (found[1] || complete)
-            row_pair(q10, 1);
-        if (found[2] || complete)
-            row_pair(q01, 2);
-        if (complete)
-            row_pair(q11, 3);
-        // case-corner order 1, 4, 3, 2, 5, 6, 7: (x+1,y,z), (x,y+1,z), (x,y,z+1), (x+1,y,z+1),
-        // (x+1,y+1,z), (x+1,y+1,z+1), (x,y+1,z+1)
-        const V cv[7] = { vrow[0][1], vrow[1][0], vrow[2][0], vrow[2][1], vrow[1][1], vrow[3][1], vrow[3][0] };
-        const bool below_g = vg < iso;
-        bool below[7];
-#pragma unroll
-        for (int k = 0; k < 7; ++k)
-            below[k] = (k < 3 ? found[k] : complete) && cv[k] < iso;
-        uint32_t sc = 0u;
-#pragma unroll
-        for (int d = 0; d < 3; ++d)
-            if (found[d] && below[d] != below_g)
-                sc |= 1u << d;
-        uint32_t ci = 0u; // missing corner or boundary vertex: cubeindex 0 (MC:206-211)
-        if (complete)
-        {
-            ci = below_g ? 1u : 0u;
-#pragma unroll
-            for (int k = 0; k < 7; ++k)
-                ci |= below[k] ? (1u << corner[k]) : 0u;
-        }
-        info = ci | (complete ? kInfoComplete : 0u) | (sc << kInfoSignShift);
-        ntv = complete ? uint32_t(c_cases.count[ci]) : 0u;
+        const pair_t v2 = *(global_pair_t*)(vals + i); // i + 1 < nverts
+        vg = v2.x;
+        vrow[0][1] = v2.y;
     }
     else
+        vg = vals[i];
+    const auto row_pair = [&](const RowProbe& q, int row) {
+        const uint32_t b = r.x & 31u;
+        const uint32_t r0 = q.pre + __popc(q.word & ((1u << b) - 1u));
+        const uint32_t a = min(r0, last2);
+        const pair_t v2 = *(global_pair_t*)(vals + a);
+        vrow[row][0] = a == r0 ? v2.x : v2.y;
+        vrow[row][1] = v2.y;
+    };
+    if (found[1] || complete)
+        row_pair(q10, 1);
+    if (found[2] || complete)
+        row_pair(q01, 2);
+    if (complete)
+        row_pair(q11, 3);
+    // case-corner order 1, 4, 3, 2, 5, 6, 7: (x+1,y,z), (x,y+1,z), (x,y,z+1), (x+1,y,z+1),
+    // (x+1,y+1,z), (x+1,y+1,z+1), (x,y+1,z+1)
+    const V cv[7] = { vrow[0][1], vrow[1][0], vrow[2][0], vrow[2][1], vrow[1][1], vrow[3][1], vrow[3][0] };
+    const bool below_g = vg < iso;
+    bool below[7];
+#pragma unroll
+    for (int k = 0; k < 7; ++k)
+        below[k] = (k < 3 ? found[k] : complete) && cv[k] < iso;
+    uint32_t sc = 0u;
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+        if (found[d] && below[d] != below_g)
+            sc |= 1u << d;
+    uint32_t ci = 0u; // missing corner or boundary vertex: cubeindex 0 (MC:206-211)
+    if (complete)
     {
-        const bool below_g = value_at<V>(p, uint32_t(i)) < iso;
-        typename Lookup::Probe pr[7];
-        cell_corners(lk, g, i, r, found, pr, inx, iny, inz);
-        bool complete = inx && iny && inz; // MC:199
+        ci = below_g ? 1u : 0u;
 #pragma unroll
         for (int k = 0; k < 7; ++k)
-            complete = complete && found[k];
-        // values: the axis neighbours when present, the other corners of a complete cell
-#pragma unroll
-        for (int k = 0; k < 7; ++k)
-            if (k < 3 ? found[k] : complete)
-                pos[k] = lk.rank(pr[k]);
-        bool below[7];
-#pragma unroll
-        for (int k = 0; k < 7; ++k)
-            below[k] = (k < 3 ? found[k] : complete) && value_at<V>(p, pos[k]) < iso;
-        uint32_t sc = 0u;
-#pragma unroll
-        for (int d = 0; d < 3; ++d)
-            if (found[d] && below[d] != below_g)
-                sc |= 1u << d;
-        uint32_t ci = 0u; // missing corner or boundary vertex: cubeindex 0 (MC:206-211)
-        if (complete)
-        {
-            ci = below_g ? 1u : 0u;
-#pragma unroll
-            for (int k = 0; k < 7; ++k)
-                ci |= below[k] ? (1u << corner[k]) : 0u;
-        }
-        info = ci | (complete ? kInfoComplete : 0u) | (sc << kInfoSignShift);
-        ntv = complete ? uint32_t(c_cases.count[ci]) : 0u;
+            ci |= below[k] ? (1u << corner[k]) : 0u;
     }
+    info = ci | (complete ? kInfoComplete : 0u) | (sc << kInfoSignShift);
+    ntv = complete ? uint32_t(c_cases.count[ci]) : 0u;
 }
 
-template <typename Lookup, typename V>
+template <typename V>
 __global__ __launch_bounds__(256) void
-mc_classify_kernel(McPlan p, Lookup lk, uint32_t* __restrict__ info, uint32_t* __restrict__ ntv)
+mc_classify_kernel(McPlan p, BitmapLookup lk, uint32_t* __restrict__ info, uint32_t* __restrict__ ntv)
 {
     const uint64_t i = uint64_t(xcd_block(blockIdx.x, gridDim.x)) * 256 + threadIdx.x;
     if (i >= p.nverts)
@@ -393,9 +294,9 @@ mc_classify_kernel(McPlan p, Lookup lk, uint32_t* __restrict__ info, uint32_t* _
     const uint32_t s0 = __builtin_amdgcn_readfirstlane(r.scene);
     uint32_t inf, n;
     if (__all(r.scene == s0)) // one grid for the whole wave: scalar grid parameters
-        mc_classify_vertex<Lookup, V, true>(p, lk, wave_uniform(p.grids[s0]), i, r, inf, n);
+        mc_classify_vertex<V, true>(p, lk, wave_uniform(p.grids[s0]), i, r, inf, n);
     else
-        mc_classify_vertex<Lookup, V, false>(p, lk, p.grids[r.scene], i, r, inf, n);
+        mc_classify_vertex<V, false>(p, lk, p.grids[r.scene], i, r, inf, n);
     info[i] = inf;
     ntv[i] = n;
 }
@@ -406,9 +307,9 @@ mc_classify_kernel(McPlan p, Lookup lk, uint32_t* __restrict__ info, uint32_t* _
 
 // Emitted edges of a vertex with sign-change bits sc (info word inf).
 // UNIFORM as for mc_classify_vertex: keeps the wave-uniform and per-lane copies apart.
-template <typename Lookup, bool UNIFORM>
+template <bool UNIFORM>
 __device__ __forceinline__ uint32_t
-mc_vertex_emask(const McPlan& p, const Lookup& lk, const McGrid& g, const uint32_t* __restrict__ info,
+mc_vertex_emask(const McPlan& p, const BitmapLookup& lk, const McGrid& g, const uint32_t* __restrict__ info,
                 const VertexRef& r, uint32_t inf, uint32_t sc)
 {
     if (inf & kInfoComplete) // the vertex's own cell is complete: every sign-changing edge is emitted
@@ -426,7 +327,7 @@ mc_vertex_emask(const McPlan& p, const Lookup& lk, const McGrid& g, const uint32
         need |= 0b011010u;
     if (sc & 4u)
         need |= 0b101001u;
-    typename Lookup::Probe pr[6];
+    BitmapLookup::Probe pr[6];
     bool ok[6];
 #pragma unroll
     for (int k = 0; k < 6; ++k)
@@ -457,25 +358,26 @@ mc_vertex_emask(const McPlan& p, const Lookup& lk, const McGrid& g, const uint32
     return m;
 }
 
-template <typename Lookup>
 __global__ __launch_bounds__(256) void
-mc_edges_kernel(McPlan p, Lookup lk, const uint32_t* __restrict__ info, uint32_t* __restrict__ emask)
+mc_edges_kernel(McPlan p, BitmapLookup lk, const uint32_t* __restrict__ info, uint32_t* __restrict__ emask)
 {
     const uint64_t i = uint64_t(xcd_block(blockIdx.x, gridDim.x)) * 256 + threadIdx.x;
     if (i >= p.nverts)
         return;
-    // the vertex's own reads are issued together, ahead of the sign-change test
+    // the vertex's own reads are issued together, ahead of the sign-change test (the empty asm keeps the
+    // compiler from moving the key's read behind the test: 62 instead of 57 us on 24 mixed scenes)
     const uint32_t inf = info[i];
-    const VertexRef r = vertex_ref(p, i);
+    VertexRef r = vertex_ref(p, i);
+    asm volatile("" : "+v"(r.scene), "+v"(r.x), "+v"(r.y), "+v"(r.z));
     const uint32_t sc = (inf >> kInfoSignShift) & 7u;
     uint32_t m = 0u;
     if (sc != 0u)
     {
         const uint32_t s0 = __builtin_amdgcn_readfirstlane(r.scene);
         if (__all(r.scene == s0)) // one grid for the active lanes: scalar grid parameters
-            m = mc_vertex_emask<Lookup, true>(p, lk, wave_uniform(p.grids[s0]), info, r, inf, sc);
+            m = mc_vertex_emask<true>(p, lk, wave_uniform(p.grids[s0]), info, r, inf, sc);
         else
-            m = mc_vertex_emask<Lookup, false>(p, lk, p.grids[r.scene], info, r, inf, sc);
+            m = mc_vertex_emask<false>(p, lk, p.grids[r.scene], info, r, inf, sc);
     }
     emask[i] = m;
 }
@@ -491,25 +393,24 @@ constexpr int kMcWaves = 256 / 64;
 
 // Output vertices of the emitted edges m of vertex i into out (3 floats each).
 // UNIFORM as for mc_classify_vertex: keeps the wave-uniform and per-lane copies apart.
-template <typename Lookup, typename V, bool UNIFORM>
+template <typename V, bool UNIFORM>
 __device__ __forceinline__ void
-mc_edge_vertices(const McPlan& p, const Lookup& lk, const McGrid& g, uint64_t i, const VertexRef& r, uint32_t m,
+mc_edge_vertices(const McPlan& p, const BitmapLookup& lk, const McGrid& g, uint64_t i, const VertexRef& r, uint32_t m,
                  float v1, float* out)
 {
     const uint32_t p1[3] = { r.x, r.y, r.z };
     // the far endpoints of the emitted edges (present: each edge has a sign change); reads batched
-    // (bitmap policy: the +x endpoint of a present vertex i is vertex i + 1)
-    constexpr bool kBitmap = std::is_same_v<Lookup, BitmapLookup>;
-    typename Lookup::Probe pr[3];
+    // (the +x endpoint of a present vertex i is vertex i + 1)
+    BitmapLookup::Probe pr[3];
 #pragma unroll
-    for (int d = kBitmap ? 1 : 0; d < 3; ++d)
+    for (int d = 1; d < 3; ++d)
         if (m & (1u << d))
             pr[d] = lk.probe(g, r.x + (d == 0), r.y + (d == 1), r.z + (d == 2));
     float v2[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d)
         if (m & (1u << d))
-            v2[d] = float(value_at<V>(p, (kBitmap && d == 0) ? uint32_t(i) + 1u : lk.rank(pr[d])));
+            v2[d] = float(value_at<V>(p, d == 0 ? uint32_t(i) + 1u : lk.rank(pr[d])));
     uint32_t o = 0u;
 #pragma unroll
     for (int d = 0; d < 3; ++d)
@@ -566,9 +467,9 @@ mc_dequeue64(McQueue& Q, uint32_t q)
 }
 
 // Output vertices of the first nb queued vertices (nb >= 1).
-template <typename Lookup, typename V>
+template <typename V>
 __device__ __forceinline__ void
-mc_vertices_batch(const McPlan& p, const Lookup& lk, const McQueue& Q, uint32_t nb,
+mc_vertices_batch(const McPlan& p, const BitmapLookup& lk, const McQueue& Q, uint32_t nb,
                   const uint32_t* __restrict__ emask, const uint32_t* __restrict__ vbase, float* __restrict__ verts,
                   float* stage)
 {
@@ -590,9 +491,9 @@ mc_vertices_batch(const McPlan& p, const Lookup& lk, const McQueue& Q, uint32_t 
         const uint32_t s0 = __builtin_amdgcn_readfirstlane(r.scene);
         float* o = stage + 3 * (out - V0);
         if (__all(r.scene == s0)) // one grid for the active lanes: scalar grid parameters
-            mc_edge_vertices<Lookup, V, true>(p, lk, wave_uniform(p.grids[s0]), i, r, m, v1, o);
+            mc_edge_vertices<V, true>(p, lk, wave_uniform(p.grids[s0]), i, r, m, v1, o);
         else
-            mc_edge_vertices<Lookup, V, false>(p, lk, p.grids[r.scene], i, r, m, v1, o);
+            mc_edge_vertices<V, false>(p, lk, p.grids[r.scene], i, r, m, v1, o);
     }
     wave_lds_sync();
     const uint32_t nf = 3u * (end - V0);
@@ -602,9 +503,9 @@ mc_vertices_batch(const McPlan& p, const Lookup& lk, const McQueue& Q, uint32_t 
     wave_lds_sync();
 }
 
-template <typename Lookup, typename V>
+template <typename V>
 __global__ __launch_bounds__(256) void
-mc_vertices_kernel(McPlan p, Lookup lk, int chunks, const uint32_t* __restrict__ emask,
+mc_vertices_kernel(McPlan p, BitmapLookup lk, int chunks, const uint32_t* __restrict__ emask,
                    const uint32_t* __restrict__ vbase, float* __restrict__ verts)
 {
     __shared__ float stage[kMcWaves][64 * 3 * 3];
@@ -623,14 +524,14 @@ mc_vertices_kernel(McPlan p, Lookup lk, int chunks, const uint32_t* __restrict__
         if (q >= 64u)
         {
             wave_lds_sync();
-            mc_vertices_batch<Lookup, V>(p, lk, queue[wave], 64u, emask, vbase, verts, stage[wave]);
+            mc_vertices_batch<V>(p, lk, queue[wave], 64u, emask, vbase, verts, stage[wave]);
             q = mc_dequeue64(queue[wave], q);
         }
     }
     if (q > 0u)
     {
         wave_lds_sync();
-        mc_vertices_batch<Lookup, V>(p, lk, queue[wave], q, emask, vbase, verts, stage[wave]);
+        mc_vertices_batch<V>(p, lk, queue[wave], q, emask, vbase, verts, stage[wave]);
     }
 }
 
@@ -638,10 +539,10 @@ mc_vertices_kernel(McPlan p, Lookup lk, int chunks, const uint32_t* __restrict__
 // Pass 4: faces (and soup vertices)
 // ---------------------------------------------------------------------------
 
-template <typename Lookup, typename V>
+template <typename V>
 __global__ __launch_bounds__(256) void
 mc_faces_kernel(McPlan p,
-                Lookup lk,
+                BitmapLookup lk,
                 const uint32_t* __restrict__ info,
                 const uint32_t* __restrict__ tbase,
                 const uint32_t* __restrict__ emask,
@@ -717,106 +618,100 @@ mc_max_case_count()
 }
 static_assert(mc_max_case_count() <= kMcMaxTriVerts, "face staging holds kMcMaxTriVerts slots per cell");
 
-// Vertex indices of the triangle corners of complete cell i (case ci, count corners) into out.
-// UNIFORM as for mc_classify_vertex: keeps the wave-uniform and per-lane copies apart.
-template <typename Lookup, bool UNIFORM>
+// Vertex indices v[0 .. count) of the triangle corners of a cell of case ci, from the vertex base vb and edge
+// mask em of its corners (meaningful where the corner is the lower endpoint of one of the case's edges).  The
+// indices of the cell's 12 edges go to the lane's row of an LDS table first, which the triangle corners then
+// pick from: selecting each corner's base and mask from the 8 registers took 36 VALU instructions per triangle
+// corner, and every lane of a batch runs as many corners as the largest cell.  Faces
+// of 24 mixed scenes: 138 -> 123 us, of a 400^3 sphere band 29 -> 25, of a level-7 hull 7.7 -> 5.7.
+constexpr uint32_t kMcEdgeRow = 13; // odd: the lanes' rows start in different banks
+static_assert(kMcEdgeRow <= kMcMaxTriVerts, "the edge table and the face staging share their LDS");
+
 __device__ __forceinline__ void
-mc_cell_faces(const McPlan& p, const Lookup& lk, const McGrid& g, uint64_t i, const VertexRef& r, uint32_t ci,
+case_faces(uint32_t ci, int count, uint32_t vs, const uint32_t (&vb)[8], const uint32_t (&em)[8], uint32_t* lds,
+           uint32_t (&v)[kMcMaxTriVerts])
+{
+    uint32_t* row = lds + (threadIdx.x & 63u) * kMcEdgeRow;
+    // the case's edges, all 15 in one 16-byte read
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const u32x4 ids = *reinterpret_cast<const u32x4*>(&c_cases.edges[ci][0]);
+    const uint32_t id[4] = { ids.x, ids.y, ids.z, ids.w };
+#pragma unroll
+    for (int e = 0; e < 12; ++e)
+        row[e] = vb[kMcEdgeLow[e]] + __popc(em[kMcEdgeLow[e]] & ((1u << kMcEdgeAxis[e]) - 1u)) - vs;
+#pragma unroll
+    for (int k = 0; k < kMcMaxTriVerts; ++k)
+        if (k - k % 3 < count)
+            v[k] = row[(id[k >> 2] >> (8 * (k & 3))) & 0xffu];
+}
+
+// The indices to the lane's slots `out` of the staging that shares its LDS with the edge tables; every lane of the
+// wavefront has read its table before.  flip_faces swaps columns 1 and 2 (visual_hull_cuda.cu:951-954).
+__device__ __forceinline__ void
+stage_faces(int count, bool flip, const uint32_t (&v)[kMcMaxTriVerts], uint32_t* out)
+{
+#pragma unroll
+    for (int t = 0; t < kMcMaxTriVerts; t += 3)
+        if (t < count)
+        {
+            out[t] = v[t];
+            out[t + 1] = flip ? v[t + 2] : v[t + 1];
+            out[t + 2] = flip ? v[t + 1] : v[t + 2];
+        }
+}
+
+// Vertex indices of the triangle corners of complete cell i (case ci, count corners).
+// UNIFORM as for mc_classify_vertex: keeps the wave-uniform and per-lane copies apart.
+template <bool UNIFORM>
+__device__ __forceinline__ void
+mc_cell_faces(const McPlan& p, const BitmapLookup& lk, const McGrid& g, uint64_t i, const VertexRef& r, uint32_t ci,
               int count, uint32_t vs, const uint32_t* __restrict__ emask, const uint32_t* __restrict__ vbase,
-              uint32_t* out)
+              uint32_t* lds, uint32_t (&v)[kMcMaxTriVerts])
 {
     // vertex base and edge mask of every corner that is the lower endpoint of one of the case's
     // edges (corner 0 is this vertex); all corners of a complete cell are present, reads batched
     const uint32_t lows = c_cases.lows[ci];
-    uint32_t vb[8], em[8];
-    if constexpr (std::is_same_v<Lookup, BitmapLookup>)
-    {
-        // corners 2q and 2q + 1 (x and x + 1) of row q = (dy, dz) are consecutive present
-        // vertices: one bitmap word and prefix give the row's rank, and the two corners' vertex
-        // bases and edge masks are read as pairs (element-aligned 8-byte loads)
-        typedef uint32_t pair_t __attribute__((ext_vector_type(2), aligned(4)));
-        typedef __attribute__((address_space(1))) const pair_t global_pair_t;
-        uint32_t pos[4];
-        pos[0] = uint32_t(i);
-        uint64_t w[4];
-        uint32_t word[4];
-        const uint32_t b = r.x & 31u;
+    uint32_t vb[8] = {}, em[8] = {};
+    // corners 2q and 2q + 1 (x and x + 1) of row q = (dy, dz) are consecutive present
+    // vertices: one bitmap word and prefix give the row's rank, and the two corners' vertex
+    // bases and edge masks are read as pairs (element-aligned 8-byte loads)
+    typedef uint32_t pair_t __attribute__((ext_vector_type(2), aligned(4)));
+    typedef __attribute__((address_space(1))) const pair_t global_pair_t;
+    uint32_t pos[4];
+    pos[0] = uint32_t(i);
+    uint64_t w[4];
+    uint32_t word[4];
+    const uint32_t b = r.x & 31u;
 #pragma unroll
-        for (int q = 1; q < 4; ++q)
-            if (lows & (3u << (2 * q)))
-            {
-                w[q] = g.bitmap_offset + (uint64_t(r.z + (q >> 1)) * g.dims[1] + (r.y + (q & 1))) * g.row_words +
-                       (r.x >> 5);
-                word[q] = lk.bitmap[w[q]];
-            }
+    for (int q = 1; q < 4; ++q)
+        if (lows & (3u << (2 * q)))
+        {
+            w[q] = g.bitmap_offset + (uint64_t(r.z + (q >> 1)) * g.dims[1] + (r.y + (q & 1))) * g.row_words +
+                   (r.x >> 5);
+            word[q] = lk.bitmap[w[q]];
+        }
 #pragma unroll
-        for (int q = 1; q < 4; ++q)
-            if (lows & (3u << (2 * q)))
-                pos[q] = lk.prefix[w[q]] + __popc(word[q] & ((1u << b) - 1u));
+    for (int q = 1; q < 4; ++q)
+        if (lows & (3u << (2 * q)))
+            pos[q] = lk.prefix[w[q]] + __popc(word[q] & ((1u << b) - 1u));
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            if (lows & (3u << (2 * q)))
-            {
-                const pair_t v2 = *(global_pair_t*)(vbase + pos[q]);
-                const pair_t e2 = *(global_pair_t*)(emask + pos[q]);
-                vb[2 * q] = v2.x;
-                vb[2 * q + 1] = v2.y;
-                em[2 * q] = e2.x;
-                em[2 * q + 1] = e2.y;
-            }
-    }
-    else
-    {
-        uint32_t pos[8];
-        pos[0] = uint32_t(i);
-        typename Lookup::Probe pr[8];
-#pragma unroll
-        for (int o = 1; o < 8; ++o)
-            if (lows & (1u << o))
-                pr[o] = lk.probe(g, r.x + (o & 1), r.y + ((o >> 1) & 1), r.z + ((o >> 2) & 1));
-#pragma unroll
-        for (int o = 1; o < 8; ++o)
-            if (lows & (1u << o))
-                pos[o] = lk.rank(pr[o]);
-#pragma unroll
-        for (int o = 0; o < 8; ++o)
-            if (lows & (1u << o))
-            {
-                vb[o] = vbase[pos[o]];
-                em[o] = emask[pos[o]];
-            }
-    }
-    // the case's edges as (lower endpoint, axis) codes, all 15 in one 16-byte read
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    const u32x4 la = *reinterpret_cast<const u32x4*>(&c_cases.low_axis[ci][0]);
-    const uint32_t law[4] = { la.x, la.y, la.z, la.w };
-#pragma unroll
-    for (int k = 0; k < kMcMaxTriVerts; ++k)
-    {
-        if (k >= count)
-            break;
-        const uint32_t code = (law[k >> 2] >> (8 * (k & 3))) & 0xffu;
-        const uint32_t lo = code >> 2, axis = code & 3u;
-        uint32_t bv = 0u, m = 0u;
-#pragma unroll
-        for (int o = 0; o < 8; ++o)
-            if (lo == uint32_t(o))
-            {
-                bv = vb[o];
-                m = em[o];
-            }
-        int col = k % 3;
-        if (g.flip && col != 0)
-            col = 3 - col; // flip_faces swaps columns 1 and 2 (visual_hull_cuda.cu:951-954)
-        out[k - k % 3 + col] = bv + __popc(m & ((1u << axis) - 1u)) - vs;
-    }
+    for (int q = 0; q < 4; ++q)
+        if (lows & (3u << (2 * q)))
+        {
+            const pair_t v2 = *(global_pair_t*)(vbase + pos[q]);
+            const pair_t e2 = *(global_pair_t*)(emask + pos[q]);
+            vb[2 * q] = v2.x;
+            vb[2 * q + 1] = v2.y;
+            em[2 * q] = e2.x;
+            em[2 * q + 1] = e2.y;
+        }
+    case_faces(ci, count, vs, vb, em, lds, v);
 }
 
 // Faces of the first nb queued complete cells (nb >= 1).
-template <typename Lookup>
 __device__ __forceinline__ void
-mc_faces_batch(const McPlan& p, const Lookup& lk, const McQueue& Q, uint32_t nb, const uint32_t* __restrict__ info,
-               const uint32_t* __restrict__ tbase, const uint32_t* __restrict__ emask,
+mc_faces_batch(const McPlan& p, const BitmapLookup& lk, const McQueue& Q, uint32_t nb,
+               const uint32_t* __restrict__ info, const uint32_t* __restrict__ tbase, const uint32_t* __restrict__ emask,
                const uint32_t* __restrict__ vbase, const uint32_t* __restrict__ scene_vstart,
                int64_t* __restrict__ faces, uint32_t* stage)
 {
@@ -834,17 +729,22 @@ mc_faces_batch(const McPlan& p, const Lookup& lk, const McQueue& Q, uint32_t nb,
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1)
         end = max(end, __shfl_xor(end, d, 64));
+    uint32_t v[kMcMaxTriVerts];
+    bool flip = false;
     if (on)
     {
         const uint32_t s0 = __builtin_amdgcn_readfirstlane(r.scene);
-        uint32_t* o = stage + (t0 - T0);
+        flip = p.grids[r.scene].flip != 0;
         if (__all(r.scene == s0)) // one grid for the active lanes: scalar grid parameters
-            mc_cell_faces<Lookup, true>(p, lk, wave_uniform(p.grids[s0]), i, r, ci, count,
-                                        __builtin_amdgcn_readfirstlane(scene_vstart[s0]), emask, vbase, o);
+            mc_cell_faces<true>(p, lk, wave_uniform(p.grids[s0]), i, r, ci, count,
+                                __builtin_amdgcn_readfirstlane(scene_vstart[s0]), emask, vbase, stage, v);
         else
-            mc_cell_faces<Lookup, false>(p, lk, p.grids[r.scene], i, r, ci, count, scene_vstart[r.scene], emask,
-                                         vbase, o);
+            mc_cell_faces<false>(p, lk, p.grids[r.scene], i, r, ci, count, scene_vstart[r.scene], emask, vbase, stage,
+                                 v);
     }
+    wave_lds_sync();
+    if (on)
+        stage_faces(count, flip, v, stage + (t0 - T0));
     wave_lds_sync();
     const uint32_t n = end - T0;
     int64_t* dst = faces + uint64_t(T0);
@@ -854,10 +754,9 @@ mc_faces_batch(const McPlan& p, const Lookup& lk, const McQueue& Q, uint32_t nb,
 }
 
 // The complete cells with triangles are gathered like the vertices of mc_vertices_kernel.
-template <typename Lookup>
 __global__ __launch_bounds__(256) void
 mc_faces_unique_kernel(McPlan p,
-                       Lookup lk,
+                       BitmapLookup lk,
                        int chunks,
                        const uint32_t* __restrict__ info,
                        const uint32_t* __restrict__ tbase,
@@ -882,16 +781,479 @@ mc_faces_unique_kernel(McPlan p,
         if (q >= 64u)
         {
             wave_lds_sync();
-            mc_faces_batch<Lookup>(p, lk, queue[wave], 64u, info, tbase, emask, vbase, scene_vstart, faces,
-                                   stage[wave]);
+            mc_faces_batch(p, lk, queue[wave], 64u, info, tbase, emask, vbase, scene_vstart, faces, stage[wave]);
             q = mc_dequeue64(queue[wave], q);
         }
     }
     if (q > 0u)
     {
         wave_lds_sync();
-        mc_faces_batch<Lookup>(p, lk, queue[wave], q, info, tbase, emask, vbase, scene_vstart, faces, stage[wave]);
+        mc_faces_batch(p, lk, queue[wave], q, info, tbase, emask, vbase, scene_vstart, faces, stage[wave]);
     }
+}
+
+// ---------------------------------------------------------------------------
+// Dense volumes (MC:146-178, MC:242-306, MC:376-533)
+//
+// Every grid point of a dense volume is present, so which edges are emitted and which case a cell has
+// follows from one bit per point: whether its value is below the isolevel.  The volume is read once into
+// that bitmap (rows padded to 32-bit words), and the rest of the work is done on words of 32 points: the
+// sign-changing edges of a word are the XOR of it with the words one step along x, y and z (every edge of a
+// volume of at least 2 points per axis belongs to a cell, so all of them are emitted), the cells with
+// triangles are those whose 8 corner bits differ.  The words' counts of output vertices and triangle
+// vertices are scanned in tiles of kDenseTile words, and the two output passes visit the words with a count
+// only: a vertex of the mesh has the index of its edge in the order (point, axis), which is its word's
+// first vertex plus three popcounts.
+//
+// A 500^3 float32 volume moves 0.5 GB once (the sign pass) and about 60 MB of words; with five 32-bit values
+// per grid point, as the sparse passes keep them, it moved 6 GB.  500^3: 2.53 ms -> 0.28 ms (the sign pass
+// 0.10 ms at 5.1 TB/s, counts 0.03, vertices 0.04, faces 0.07); 61 x 83 x 71 float64: 85 -> 54 us.
+// ---------------------------------------------------------------------------
+
+// Words per workgroup of the counting pass (one per thread) and per entry of the scanned
+// tile counts.
+constexpr int kDenseTile = 256;
+
+// Edge masks of a word's 32 points along x, y and z, and the index of its first output vertex (written by
+// the vertex pass).  Words that emit no edge have no record.
+struct alignas(16) DenseEdges
+{
+    uint32_t x, y, z, first;
+};
+
+// A word's counts: output vertices in the low byte (at most 96), triangle vertices above.
+__device__ __forceinline__ uint32_t
+dense_verts(uint32_t c)
+{
+    return c & 0xffu;
+}
+__device__ __forceinline__ uint32_t
+dense_tris(uint32_t c)
+{
+    return c >> 8;
+}
+
+// Sign bits.  A lane reads 4 consecutive points in each of kSignRows consecutive rows (16-byte loads of
+// float32, element-aligned, all in flight together); 8 lanes assemble a word.  Bound by the one read of the
+// volume.
+constexpr int kSignRows = 4;
+
+template <typename V>
+__global__ __launch_bounds__(256) void
+mc_dense_signs_kernel(const V* __restrict__ volume, uint32_t W, uint32_t rows, uint32_t row_words, float isolevel,
+                      uint32_t* __restrict__ signs)
+{
+    typedef V quad_t __attribute__((ext_vector_type(4), aligned(sizeof(V))));
+    typedef __attribute__((address_space(1))) const quad_t global_quad_t;
+    const V iso = static_cast<V>(isolevel);
+    const uint32_t quads = row_words * 8u; // per row, a multiple of 8: the 8 lanes of a word stay together
+    const uint64_t t = uint64_t(blockIdx.x) * 256 + threadIdx.x;
+    const uint64_t r0 = div_u64_u32(t, quads) * kSignRows;
+    const uint32_t quad = uint32_t(t - (r0 / kSignRows) * quads);
+    const uint32_t x = quad * 4u;
+    const auto src = as_global(volume);
+    quad_t v[kSignRows] = {};
+    uint32_t n = 0u; // points of this lane's quad inside the row
+    if (x < W)
+        n = min(W - x, 4u);
+#pragma unroll
+    for (int q = 0; q < kSignRows; ++q)
+        if (r0 + q < rows)
+        {
+            const uint64_t at = (r0 + q) * W + x;
+            if (n == 4u)
+                v[q] = *(global_quad_t*)(src + at);
+            else
+            {
+                if (n > 0u)
+                    v[q].x = src[at];
+                if (n > 1u)
+                    v[q].y = src[at + 1];
+                if (n > 2u)
+                    v[q].z = src[at + 2];
+            }
+        }
+    const uint32_t sub = threadIdx.x & 7u, inside = (1u << n) - 1u;
+    uint32_t mine = 0u;
+#pragma unroll
+    for (int q = 0; q < kSignRows; ++q)
+    {
+        uint32_t b = (v[q].x < iso ? 1u : 0u) | (v[q].y < iso ? 2u : 0u) | (v[q].z < iso ? 4u : 0u) |
+                     (v[q].w < iso ? 8u : 0u);
+        b = (b & inside) << (4u * sub);
+        b |= uint32_t(__shfl_xor(int(b), 1, 64));
+        b |= uint32_t(__shfl_xor(int(b), 2, 64));
+        b |= uint32_t(__shfl_xor(int(b), 4, 64));
+        if (sub == uint32_t(q))
+            mine = b;
+    }
+    if (sub < uint32_t(kSignRows) && r0 + sub < rows)
+        as_global(signs)[(r0 + sub) * row_words + quad / 8u] = mine;
+}
+
+// Position of a word: row = y + z H and the points of it inside the volume.
+struct DenseWord
+{
+    uint32_t row, xw, z;
+    bool iny, inz;   // rows y + 1 and z + 1 exist
+    uint32_t points; // bits of points inside the volume
+    uint32_t stepx;  // bits of points with a +x neighbour
+};
+
+__device__ __forceinline__ DenseWord
+dense_word(const McDense& d, uint32_t w)
+{
+    DenseWord q;
+    q.row = w / d.row_words;
+    q.xw = w - q.row * d.row_words;
+    q.z = q.row / d.dims[1];
+    q.iny = q.row - q.z * d.dims[1] + 1u < d.dims[1];
+    q.inz = q.z + 1u < d.dims[2];
+    const uint32_t left = d.dims[0] - q.xw * 32u; // points of the row from this word on, at least 1
+    q.points = left >= 32u ? 0xffffffffu : (1u << left) - 1u;
+    q.stepx = left > 32u ? 0xffffffffu : q.points >> 1;
+    return q;
+}
+
+// Sign words of a word's four rows (dy, dz) = (0, 0), (1, 0), (0, 1), (1, 1) and of the points one step along
+// x from them; rows outside the volume read as the word's own (their results are masked).
+struct DenseSigns
+{
+    uint32_t s[4], x[4];
+};
+
+__device__ __forceinline__ DenseSigns
+dense_signs(const McDense& d, const DenseWord& q, uint32_t w)
+{
+    const auto S = as_global(d.signs);
+    const uint32_t next = q.xw + 1u < d.row_words ? 1u : 0u;
+    const uint32_t oy = q.iny ? d.row_words : 0u, oz = q.inz ? d.row_words * d.dims[1] : 0u;
+    DenseSigns g;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+    {
+        const uint32_t at = w + ((r & 1) ? oy : 0u) + ((r >> 1) ? oz : 0u);
+        g.s[r] = S[at];
+        g.x[r] = S[at + next];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        g.x[r] = (g.s[r] >> 1) | (g.x[r] << 31);
+    return g;
+}
+
+// Cells of the word with triangles: complete cells whose corners differ.
+__device__ __forceinline__ uint32_t
+dense_active(const DenseWord& q, const DenseSigns& g)
+{
+    uint32_t any = 0u, all = 0xffffffffu;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+    {
+        any |= g.s[r] | g.x[r];
+        all &= g.s[r] & g.x[r];
+    }
+    return (q.iny && q.inz) ? (any & ~all & q.stepx) : 0u;
+}
+
+// Case of the cell at bit b: case corner k is the point at offset c_corner_off[k].
+__device__ __forceinline__ uint32_t
+dense_case(const DenseSigns& g, uint32_t b)
+{
+    uint32_t ci = 0u;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+    {
+        const int o = c_corner_off_host[k];
+        ci |= ((((o & 1) ? g.x[o >> 1] : g.s[o >> 1]) >> b) & 1u) << k;
+    }
+    return ci;
+}
+
+// Edge masks and counts of every word, and the sums of each tile of words.
+__global__ __launch_bounds__(256) void
+mc_dense_count_kernel(McDense d, DenseEdges* __restrict__ edges, uint32_t* __restrict__ counts,
+                      uint32_t* __restrict__ tile_verts, uint32_t* __restrict__ tile_tris)
+{
+    __shared__ uint8_t case_count[256];
+    __shared__ uint32_t sums[2];
+    case_count[threadIdx.x] = c_cases.count[threadIdx.x];
+    if (threadIdx.x < 2)
+        sums[threadIdx.x] = 0u;
+    __syncthreads();
+    const uint64_t wl = uint64_t(blockIdx.x) * kDenseTile + threadIdx.x;
+    uint32_t nv = 0u, nt = 0u;
+    if (wl < d.nwords)
+    {
+        const uint32_t w = uint32_t(wl);
+        const DenseWord q = dense_word(d, w);
+        const DenseSigns g = dense_signs(d, q, w);
+        DenseEdges e;
+        e.x = (g.s[0] ^ g.x[0]) & q.stepx;
+        e.y = q.iny ? (g.s[0] ^ g.s[1]) & q.points : 0u;
+        e.z = q.inz ? (g.s[0] ^ g.s[2]) & q.points : 0u;
+        e.first = 0u;
+        nv = uint32_t(__popc(e.x) + __popc(e.y) + __popc(e.z));
+        for (uint32_t act = dense_active(q, g); act != 0u; act &= act - 1u)
+            nt += case_count[dense_case(g, uint32_t(__builtin_ctz(act)))];
+        if (nv != 0u)
+            edges[w] = e;
+        counts[w] = nv | (nt << 8);
+    }
+    nv = __reduce_add_sync(0xffffffffffffffffull, nv);
+    nt = __reduce_add_sync(0xffffffffffffffffull, nt);
+    if ((threadIdx.x & 63) == 0)
+    {
+        atomicAdd(&sums[0], nv);
+        atomicAdd(&sums[1], nt);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0)
+    {
+        tile_verts[blockIdx.x] = sums[0];
+        tile_tris[blockIdx.x] = sums[1];
+    }
+}
+
+// The output passes run single wavefronts of 64 words, one per lane.
+constexpr uint32_t kDenseWaves = kDenseTile / 64;
+
+// First output of each lane's word: the tile's offset plus the counts of the tile's words before it.  `own` is
+// the lane's count, `total` the wavefront's.
+template <typename Count>
+__device__ __forceinline__ uint32_t
+dense_first(const McDense& d, const uint32_t* __restrict__ counts, const uint32_t* __restrict__ tile_first,
+            Count count, uint32_t& own, uint32_t& total)
+{
+    const uint32_t q = blockIdx.x % kDenseWaves;
+    const uint64_t w = uint64_t(blockIdx.x) * 64u + threadIdx.x;
+    uint32_t before = 0u;
+#pragma unroll
+    for (uint32_t k = 1; k < kDenseWaves; ++k)
+        before += k <= q ? count(counts[w - 64u * k]) : 0u; // words of the wavefronts before: all inside
+    own = w < d.nwords ? count(counts[w]) : 0u;
+    const uint32_t inc = wave_inclusive_sum(own);
+    total = uint32_t(__shfl(int(inc), 63, 64));
+    return tile_first[blockIdx.x / kDenseWaves] + __reduce_add_sync(0xffffffffffffffffull, before) + inc - own;
+}
+
+// The lanes' set bits, one entry (lane << 5 | bit) each, in lane order; returns their number.
+__device__ __forceinline__ uint32_t
+dense_enqueue(uint16_t* queue, uint32_t bits)
+{
+    const uint32_t n = uint32_t(__popc(bits)), inc = wave_inclusive_sum(n);
+    for (uint32_t at = inc - n; bits != 0u; bits &= bits - 1u)
+        queue[at++] = uint16_t((threadIdx.x << 5) | uint32_t(__builtin_ctz(bits)));
+    wave_lds_sync();
+    return uint32_t(__shfl(int(inc), 63, 64));
+}
+
+// Output vertices of the compact mesh.  A lane records its word's first vertex and queues its points that emit
+// an edge; the wavefront then takes the queued points 64 at a time.  Bound by the latency of the value reads.
+template <typename V>
+__global__ __launch_bounds__(64) void
+mc_dense_vertices_kernel(McDense d, McGrid g, const V* __restrict__ volume, float iso,
+                         const uint32_t* __restrict__ counts, const uint32_t* __restrict__ tile_verts,
+                         DenseEdges* __restrict__ edges, float* __restrict__ verts)
+{
+    __shared__ DenseEdges rec[64];
+    __shared__ uint16_t queue[64 * 32];
+    const uint32_t lane = threadIdx.x;
+    const uint64_t w0 = uint64_t(blockIdx.x) * 64u; // the wavefront's first word
+    uint32_t c, total;
+    const uint32_t first = dense_first(d, counts, tile_verts, dense_verts, c, total);
+    if (total == 0u)
+        return;
+    uint32_t points = 0u;
+    if (c != 0u)
+    {
+        DenseEdges r = edges[w0 + lane];
+        r.first = first;
+        edges[w0 + lane].first = first;
+        rec[lane] = r;
+        points = r.x | r.y | r.z;
+    }
+    const uint32_t n = dense_enqueue(queue, points);
+    const uint32_t step[3] = { 1u, d.dims[0], d.dims[0] * d.dims[1] };
+    for (uint32_t k = lane; k < n; k += 64)
+    {
+        const uint32_t e = queue[k], b = e & 31u, lt = (1u << b) - 1u;
+        const DenseEdges r = rec[e >> 5];
+        const DenseWord q = dense_word(d, uint32_t(w0) + (e >> 5));
+        const uint32_t x = q.xw * 32u + b, y = q.row - q.z * d.dims[1];
+        const uint32_t i = q.row * d.dims[0] + x; // fewer than 2^32 points
+        const bool on[3] = { ((r.x >> b) & 1u) != 0u, ((r.y >> b) & 1u) != 0u, ((r.z >> b) & 1u) != 0u };
+        const float v1 = float(volume[i]); // stored as float (MC:343)
+        float v2[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+            v2[a] = on[a] ? float(volume[i + step[a]]) : 0.0f;
+        uint64_t o = 3 * uint64_t(r.first + uint32_t(__popc(r.x & lt) + __popc(r.y & lt) + __popc(r.z & lt)));
+        const uint32_t p1[3] = { x, y, q.z };
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+            if (on[a])
+            {
+                const uint32_t p2[3] = { x + (a == 0), y + (a == 1), q.z + (a == 2) };
+                float v[3];
+                interpolate_vertex(iso, p1, p2, v1, v2[a], v);
+                finish_vertex(g, v, verts + o);
+                o += 3;
+            }
+    }
+}
+
+// Faces, and the vertices of a triangle soup.  As the vertex pass, with the cells that have triangles; a cell's
+// first triangle vertex is the running total of the cells before it.  The slots of 64 queued cells are one
+// contiguous range, assembled in LDS and written with coalesced stores.
+template <typename V, bool UNIQUE>
+__global__ __launch_bounds__(64) void
+mc_dense_faces_kernel(McDense d, McGrid g, const V* __restrict__ volume, float iso,
+                      const uint32_t* __restrict__ counts, const uint32_t* __restrict__ tile_tris,
+                      const DenseEdges* __restrict__ edges, float* __restrict__ soup_verts,
+                      int64_t* __restrict__ faces)
+{
+    __shared__ DenseSigns signs[64];
+    __shared__ uint16_t queue[64 * 32];
+    __shared__ uint32_t stage[UNIQUE ? 64 * kMcMaxTriVerts : 1];
+    const uint32_t lane = threadIdx.x;
+    const uint64_t w0 = uint64_t(blockIdx.x) * 64u; // the wavefront's first word
+    uint32_t c, total;
+    const uint32_t first = dense_first(d, counts, tile_tris, dense_tris, c, total);
+    if (total == 0u)
+        return;
+    uint32_t run = __builtin_amdgcn_readfirstlane(first); // first triangle vertex of the cells taken next
+    uint32_t cells = 0u;
+    if (c != 0u)
+    {
+        const DenseWord q = dense_word(d, uint32_t(w0) + lane);
+        const DenseSigns s = dense_signs(d, q, uint32_t(w0) + lane);
+        cells = dense_active(q, s);
+        signs[lane] = s;
+    }
+    const uint32_t n = dense_enqueue(queue, cells);
+    const uint32_t wy = d.row_words, wz = d.row_words * d.dims[1];
+    for (uint32_t k0 = 0; k0 < n; k0 += 64)
+    {
+        const bool on = k0 + lane < n;
+        const uint32_t e = on ? queue[k0 + lane] : 0u;
+        const uint32_t b = e & 31u, w = uint32_t(w0) + (e >> 5);
+        const uint32_t ci = on ? dense_case(signs[e >> 5], b) : 0u;
+        const int count = on ? c_cases.count[ci] : 0;
+        const uint32_t inc = wave_inclusive_sum(uint32_t(count));
+        const uint32_t off = inc - uint32_t(count); // of the cell's slots in this batch
+        const uint32_t slots = uint32_t(__shfl(int(inc), 63, 64));
+        if constexpr (UNIQUE)
+        {
+            uint32_t v[kMcMaxTriVerts];
+            if (on)
+            {
+                // corners 2q and 2q + 1 (x and x + 1) of row q = (dy, dz): same word unless x is its last point
+                const uint32_t lows = c_cases.lows[ci];
+                uint32_t vb[8], em[8];
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                {
+                    const uint32_t wq = w + ((q & 1) ? wy : 0u) + ((q >> 1) ? wz : 0u);
+                    DenseEdges r{};
+                    if (lows & ((b != 31u ? 3u : 1u) << (2 * q))) // a corner that emits an edge: its word has a record
+                        r = edges[wq];
+                    DenseEdges r1 = r;
+                    if (b == 31u && (lows & (2u << (2 * q))))
+                        r1 = edges[wq + 1u];
+                    const uint32_t b1 = (b + 1u) & 31u, lt = (1u << b) - 1u, lt1 = (1u << b1) - 1u;
+                    vb[2 * q] = r.first + uint32_t(__popc(r.x & lt) + __popc(r.y & lt) + __popc(r.z & lt));
+                    em[2 * q] = ((r.x >> b) & 1u) | (((r.y >> b) & 1u) << 1) | (((r.z >> b) & 1u) << 2);
+                    vb[2 * q + 1] = r1.first + uint32_t(__popc(r1.x & lt1) + __popc(r1.y & lt1) + __popc(r1.z & lt1));
+                    em[2 * q + 1] = ((r1.x >> b1) & 1u) | (((r1.y >> b1) & 1u) << 1) | (((r1.z >> b1) & 1u) << 2);
+                }
+                case_faces(ci, count, 0u, vb, em, stage, v);
+            }
+            wave_lds_sync();
+            if (on)
+                stage_faces(count, false, v, stage + off);
+            wave_lds_sync();
+            for (uint32_t s = lane; s < slots; s += 64)
+                faces[uint64_t(run) + s] = int64_t(stage[s]);
+            wave_lds_sync();
+        }
+        else if (on)
+        {
+            const DenseWord q = dense_word(d, w);
+            const uint32_t x = q.xw * 32u + b, y = q.row - q.z * d.dims[1];
+            const uint64_t t0 = uint64_t(run) + off;
+            for (int k = 0; k < count; ++k)
+            {
+                const int id = c_cases.edges[ci][k];
+                const uint32_t lo = c_edge_low[id], axis = c_edge_axis[id];
+                const uint32_t q1[3] = { x + (lo & 1u), y + ((lo >> 1) & 1u), q.z + ((lo >> 2) & 1u) };
+                const uint32_t q2[3] = { q1[0] + (axis == 0u), q1[1] + (axis == 1u), q1[2] + (axis == 2u) };
+                const float v1 = float(volume[(q1[2] * d.dims[1] + q1[1]) * d.dims[0] + q1[0]]);
+                const float v2 = float(volume[(q2[2] * d.dims[1] + q2[1]) * d.dims[0] + q2[0]]);
+                float v[3];
+                interpolate_vertex(iso, q1, q2, v1, v2, v);
+                finish_vertex(g, v, soup_verts + 3 * (t0 + uint32_t(k)));
+                faces[t0 + uint32_t(k)] = int64_t(t0 + uint32_t(k)); // faces = arange (MC:515-519)
+            }
+        }
+        run += slots;
+    }
+}
+
+uint32_t
+mc_dense_tiles(uint64_t nwords)
+{
+    return uint32_t((nwords + kDenseTile - 1) / kDenseTile);
+}
+
+size_t
+mc_dense_edge_bytes(uint64_t nwords)
+{
+    return size_t(nwords) * sizeof(DenseEdges);
+}
+
+void
+launch_mc_dense_counts(const McDense& d, const void* volume, int32_t value_type, float iso, void* edges,
+                       uint32_t* counts, uint32_t* tile_verts, uint32_t* tile_tris, hipStream_t st)
+{
+    const uint32_t rows = d.dims[1] * d.dims[2];
+    const uint64_t threads = uint64_t(d.row_words) * 8u * ((uint64_t(rows) + kSignRows - 1) / kSignRows);
+    const unsigned nb = unsigned((threads + 255) / 256);
+    if (value_type == kMcF64)
+        mc_dense_signs_kernel<double>
+            <<<nb, 256, 0, st>>>(static_cast<const double*>(volume), d.dims[0], rows, d.row_words, iso, d.signs);
+    else
+        mc_dense_signs_kernel<float>
+            <<<nb, 256, 0, st>>>(static_cast<const float*>(volume), d.dims[0], rows, d.row_words, iso, d.signs);
+    THULL_LAUNCH_CHECK();
+    mc_dense_count_kernel<<<mc_dense_tiles(d.nwords), 256, 0, st>>>(d, static_cast<DenseEdges*>(edges), counts,
+                                                                    tile_verts, tile_tris);
+    THULL_LAUNCH_CHECK();
+}
+
+void
+launch_mc_dense_mesh(const McDense& d, const McGrid& g, const void* volume, int32_t value_type, float iso,
+                     const uint32_t* counts, const uint32_t* tile_verts, const uint32_t* tile_tris, void* edges,
+                     bool unique, float* verts, int64_t* faces, hipStream_t st)
+{
+    const unsigned nb = unsigned((d.nwords + 63) / 64);
+    DenseEdges* e = static_cast<DenseEdges*>(edges);
+    const auto run = [&](auto* vol) {
+        using V = std::remove_const_t<std::remove_pointer_t<decltype(vol)>>;
+        if (unique)
+        {
+            mc_dense_vertices_kernel<V><<<nb, 64, 0, st>>>(d, g, vol, iso, counts, tile_verts, e, verts);
+            THULL_LAUNCH_CHECK();
+            mc_dense_faces_kernel<V, true><<<nb, 64, 0, st>>>(d, g, vol, iso, counts, tile_tris, e, verts, faces);
+        }
+        else
+            mc_dense_faces_kernel<V, false><<<nb, 64, 0, st>>>(d, g, vol, iso, counts, tile_tris, e, verts, faces);
+        THULL_LAUNCH_CHECK();
+    };
+    if (value_type == kMcF64)
+        run(static_cast<const double*>(volume));
+    else
+        run(static_cast<const float*>(volume));
 }
 
 // ---------------------------------------------------------------------------
@@ -922,22 +1284,10 @@ template <typename F>
 static void
 dispatch_mc(const McPlan& p, F&& f)
 {
-    BitmapLookup bl{ p.bitmap, p.prefix };
-    DenseLookup dl{};
-    if (p.dense)
-    {
-        if (p.value_type == kMcF64)
-            f(dl, double{});
-        else
-            f(dl, float{});
-    }
+    if (p.value_type == kMcF64)
+        f(double{});
     else
-    {
-        if (p.value_type == kMcF64)
-            f(bl, double{});
-        else
-            f(bl, float{});
-    }
+        f(float{});
 }
 
 void
@@ -945,10 +1295,10 @@ launch_mc_classify(const McPlan& p, uint32_t* info, uint32_t* ntv, hipStream_t s
 {
     if (p.nverts == 0)
         return;
-    dispatch_mc(p, [&](auto lk, auto vt) {
-        using LK = decltype(lk);
+    const BitmapLookup lk{ p.bitmap, p.prefix };
+    dispatch_mc(p, [&](auto vt) {
         using VT = decltype(vt);
-        mc_classify_kernel<LK, VT><<<blocks_for(int64_t(p.nverts), 256), 256, 0, st>>>(p, lk, info, ntv);
+        mc_classify_kernel<VT><<<blocks_for(int64_t(p.nverts), 256), 256, 0, st>>>(p, lk, info, ntv);
     });
     THULL_LAUNCH_CHECK();
 }
@@ -958,10 +1308,8 @@ launch_mc_edges(const McPlan& p, const uint32_t* info, uint32_t* emask, hipStrea
 {
     if (p.nverts == 0)
         return;
-    dispatch_mc(p, [&](auto lk, auto) {
-        using LK = decltype(lk);
-        mc_edges_kernel<LK><<<blocks_for(int64_t(p.nverts), 256), 256, 0, st>>>(p, lk, info, emask);
-    });
+    mc_edges_kernel<<<blocks_for(int64_t(p.nverts), 256), 256, 0, st>>>(p, BitmapLookup{ p.bitmap, p.prefix }, info,
+                                                                        emask);
     THULL_LAUNCH_CHECK();
 }
 
@@ -970,11 +1318,11 @@ launch_mc_vertices(const McPlan& p, const uint32_t* emask, const uint32_t* vbase
 {
     if (p.nverts == 0)
         return;
-    dispatch_mc(p, [&](auto lk, auto vt) {
-        using LK = decltype(lk);
+    const BitmapLookup lk{ p.bitmap, p.prefix };
+    dispatch_mc(p, [&](auto vt) {
         using VT = decltype(vt);
         const int chunks = mc_chunks(p.nverts, kMcVertexChunks);
-        mc_vertices_kernel<LK, VT><<<mc_gather_blocks(p.nverts, chunks), 256, 0, st>>>(p, lk, chunks, emask, vbase,
+        mc_vertices_kernel<VT><<<mc_gather_blocks(p.nverts, chunks), 256, 0, st>>>(p, lk, chunks, emask, vbase,
                                                                                       verts);
     });
     THULL_LAUNCH_CHECK();
@@ -995,15 +1343,15 @@ launch_mc_faces(const McPlan& p,
 {
     if (p.nverts == 0)
         return;
-    dispatch_mc(p, [&](auto lk, auto vt) {
-        using LK = decltype(lk);
+    const BitmapLookup lk{ p.bitmap, p.prefix };
+    dispatch_mc(p, [&](auto vt) {
         using VT = decltype(vt);
         const int chunks = mc_chunks(p.nverts, kMcFaceChunks);
         if (unique)
-            mc_faces_unique_kernel<LK><<<mc_gather_blocks(p.nverts, chunks), 256, 0, st>>>(
+            mc_faces_unique_kernel<<<mc_gather_blocks(p.nverts, chunks), 256, 0, st>>>(
                     p, lk, chunks, info, ntv_base, emask, vbase, scene_vstart, faces);
         else
-            mc_faces_kernel<LK, VT><<<blocks_for(int64_t(p.nverts), 256), 256, 0, st>>>(
+            mc_faces_kernel<VT><<<blocks_for(int64_t(p.nverts), 256), 256, 0, st>>>(
                     p, lk, info, ntv_base, emask, vbase, scene_vstart, scene_tstart, unique, soup_verts, faces);
     });
     THULL_LAUNCH_CHECK();

@@ -164,6 +164,81 @@ scan_block_sums_kernel(uint32_t* sums, uint32_t nblocks, unsigned long long* tot
     }
 }
 
+// As scan_block_sums_kernel for two arrays of n sums at once (16-byte aligned, room for n rounded up to 4);
+// the host is sent both totals (`note.extra` unused).  A thread takes a run of whole 16-byte groups.
+template <typename Tag = void>
+__global__ __launch_bounds__(1024) void
+scan_block_sums2_kernel(uint32_t* a, uint32_t* b, uint32_t n, unsigned long long* totals, ScanNotify note)
+{
+    __shared__ unsigned long long lds[2][1024 / 64];
+    const uint32_t groups = (n + 3) / 4, per = (groups + 1023) / 1024;
+    const uint32_t begin = threadIdx.x * per, end = min(begin + per, groups);
+    uint4* const v[2] = { reinterpret_cast<uint4*>(a), reinterpret_cast<uint4*>(b) };
+    // group k with the entries past n as zeros
+    const auto load = [&](int q, uint32_t k) {
+        uint4 u = v[q][k];
+        u.y = 4 * k + 1 < n ? u.y : 0u;
+        u.z = 4 * k + 2 < n ? u.z : 0u;
+        u.w = 4 * k + 3 < n ? u.w : 0u;
+        return u;
+    };
+    unsigned long long sum[2] = { 0, 0 };
+    for (uint32_t k = begin; k < end; ++k)
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+        {
+            const uint4 u = load(q, k);
+            sum[q] += (unsigned long long)u.x + u.y + u.z + u.w;
+        }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    unsigned long long inc[2] = { sum[0], sum[1] };
+    for (int d = 1; d < 64; d <<= 1)
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+        {
+            const unsigned long long o = __shfl_up(inc[q], d, 64);
+            if (lane >= d)
+                inc[q] += o;
+        }
+    if (lane == 63)
+    {
+        lds[0][wave] = inc[0];
+        lds[1][wave] = inc[1];
+    }
+    __syncthreads();
+    unsigned long long run[2], total[2] = { 0, 0 };
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+    {
+        unsigned long long off = 0;
+        for (int w = 0; w < 1024 / 64; ++w)
+        {
+            if (w < wave)
+                off += lds[q][w];
+            total[q] += lds[q][w];
+        }
+        run[q] = off + inc[q] - sum[q];
+    }
+    if (threadIdx.x == 0)
+    {
+        totals[0] = total[0];
+        totals[1] = total[1];
+        note.slot[0] = total[0];
+        note.slot[1] = total[1];
+        __hip_atomic_store(note.slot + 2, note.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    for (uint32_t k = begin; k < end; ++k)
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+        {
+            const uint4 u = load(q, k);
+            const unsigned long long r = run[q];
+            v[q][k] = make_uint4(uint32_t(r), uint32_t(r + u.x), uint32_t(r + u.x + u.y),
+                                 uint32_t(r + u.x + u.y + u.z));
+            run[q] = r + u.x + u.y + u.z + u.w;
+        }
+}
+
 template <typename L>
 __global__ __launch_bounds__(kScanThreads) void
 scan_downsweep_kernel(L load, uint64_t n, const uint32_t* block_offsets, uint32_t* out)
