@@ -272,6 +272,25 @@ integral_col_offset(uint32_t X)
 }
 
 // ---------------------------------------------------------------------------
+// Solid maps: per camera one byte per tile of 4 x 4 pixels, the Chebyshev distance in tiles (at most
+// kSolidReach) to the nearest tile that is not solid, 0 for such a tile itself.  A tile is solid when it lies
+// inside the image and all its pixels are exactly 1; what lies outside the image counts as not solid.
+// ---------------------------------------------------------------------------
+
+constexpr int kSolidTile = 4;
+constexpr int kSolidReach = 15;
+
+// Per camera: how far a carving window may reach from its cell's centre for the camera to be skipped
+// (carve_skips), and bounds of the projection's rounding errors over the scene's cube.
+struct CullCamera
+{
+    float reach;      // pixels; negative: never skipped
+    float sum_d;      // sum of the magnitudes of the denominator row's first three coefficients
+    float ex, ey, ed; // rounding errors of the two numerators and the denominator
+    float pad_[3];
+};
+
+// ---------------------------------------------------------------------------
 // Scene descriptor (device side).  One per scene of a batch.
 // ---------------------------------------------------------------------------
 
@@ -296,7 +315,19 @@ struct SceneDev
     // bitmap of leaf cells R^3 with rows padded to `cell_row_words` words
     uint32_t cell_row_words;
     uint32_t* cells;        // the scene's leaf-cell bitmap
+    // solid maps (null: none) of solid_h x solid_w tiles per camera, and one CullCamera per camera
+    const uint8_t* solid;
+    const CullCamera* cull;
+    int32_t solid_h, solid_w;
+    // field by bricks (null: not used): one bit per brick of 2^brick_shift cells per side of the scene's octree,
+    // set for the bricks among the kept cells
+    uint32_t* bricks;
+    int32_t brick_shift;
+    int32_t pad_;
 };
+
+// Bricks of the field are at most 8 cells per side.
+constexpr int kBrickShift = 3;
 
 // ---------------------------------------------------------------------------
 // Global-memory pointers.  Pointers read from a table in device memory are

@@ -764,6 +764,26 @@ check_scene(const thull_scene& sc)
                 "masks must be float32, uint8 or bool at the C ABI");
 }
 
+// Solid maps and the field by bricks cost a few launches and a sixteenth of a pass over the masks, and save camera
+// tests and samples of the scenes' surface cells, about 4^level of them in every camera: they are used from
+// kMinCellCameras cell-cameras in the scenes a run starts with (16.8 million, 64 cameras at level 9: 1.96 -> 1.60 ms;
+// 6.4 million in 10 mixed scenes: 1.66 -> 1.75; 0.7 million, 10 cameras at level 8: 0.50 -> 0.54).
+static bool
+solid_maps_pay(const thull_scene* scenes, int32_t n)
+{
+    constexpr int64_t kMinCellCameras = int64_t(1) << 23;
+    int64_t work = 0;
+    for (int32_t i = 0; i < n; ++i)
+        work += std::max<int64_t>(scenes[i].B, 0) << (2 * std::clamp(scenes[i].level, 0, 12));
+    return work >= kMinCellCameras;
+}
+
+static bool
+has_solid_map(const thull_scene& sc)
+{
+    return sc.H >= 4 * kSolidTile && sc.W >= 4 * kSolidTile && sc.B >= 3;
+}
+
 static void
 visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hipStream_t st, thull_vh_counts* counts,
                 JoinFn join, void* user, int32_t max_scenes, int32_t* n_total)
@@ -794,6 +814,7 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
     // every level's list keeps the scenes in root order, so each carving launch starts with its most
     // expensive cells and ends with the cheapest ones instead of finishing on a tail of many-camera
     // cells.  Each scene's own cells keep the reference's parent-major order, so no result depends on it.
+    const bool by_bricks = solid_maps_pay(in, n0);
     auto add_scenes = [&](size_t k0, int32_t start) {
         const size_t k1 = all.size();
         std::vector<IntegralRequest> ireq;
@@ -834,14 +855,40 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
             {
                 float* integral = pool.alloc<float>(uint64_t(sc.B) * uint64_t(integral_rows(sc.H)) *
                                                     uint64_t(integral_pitch(sc.W)));
-                ireq.push_back(IntegralRequest{ sc.masks, sc.mask_dtype, sc.B, sc.H, sc.W, integral });
+                IntegralRequest r{ sc.masks, sc.mask_dtype, sc.B, sc.H, sc.W, integral };
                 d.integral = integral;
+                if (by_bricks && has_solid_map(sc))
+                {
+                    r.solid = pool.alloc<uint8_t>(solid_map_bytes(sc.B, sc.H, sc.W));
+                    r.cull = pool.alloc<CullCamera>(uint64_t(sc.B));
+                    r.solid_scratch = pool.alloc_bytes(solid_scratch_bytes(sc.B, sc.H, sc.W));
+                    r.transforms = sc.transforms;
+                    r.opengl = sc.opengl;
+                    std::copy(sc.cube_corner_bfl, sc.cube_corner_bfl + 3, r.corner);
+                    r.length = sc.cube_length;
+                    d.solid = r.solid;
+                    d.cull = r.cull;
+                    d.solid_h = int32_t(sc.H / kSolidTile);
+                    d.solid_w = int32_t(sc.W / kSolidTile);
+                }
+                ireq.push_back(r);
             }
             sd.push_back(d);
         }
-        // leaf-cell bitmaps, filled by the scatter of each scene's last carving step
-        uint32_t* cells = pool.alloc<uint32_t>(std::max<uint64_t>(cell_words, 1));
-        launch_fill_u32(cells, cell_words, 0u, st);
+        // brick bitmaps, and leaf-cell bitmaps, filled by the scatter of each scene's last carving step
+        uint64_t brick_words = 0;
+        for (size_t s = k0; by_bricks && s < k1; ++s)
+        {
+            sd[s].brick_shift = std::min(kBrickShift, sd[s].level);
+            brick_words += ((uint64_t(1) << (3 * (sd[s].level - sd[s].brick_shift))) + 31) / 32;
+        }
+        uint32_t* cells = pool.alloc<uint32_t>(std::max<uint64_t>(cell_words + brick_words, 1));
+        launch_fill_u32(cells, cell_words + brick_words, 0u, st);
+        for (size_t s = k0, w = cell_words; by_bricks && s < k1; ++s)
+        {
+            sd[s].bricks = cells + w;
+            w += ((size_t(1) << (3 * (sd[s].level - sd[s].brick_shift))) + 31) / 32;
+        }
         if (k0 == 0)
         {
             first_cells = cells;
@@ -858,8 +905,8 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
             carry_floats += integral_carry_floats(r.B, r.H, r.W);
         launch_integral_images_padded(ireq.data(), int32_t(ireq.size()),
                                       pool.alloc<float>(std::max<uint64_t>(carry_floats, 1)),
-                                      pool.alloc_bytes(integral_job_bytes(std::max<size_t>(ireq.size(), 1))), ctx.upload,
-                                      st);
+                                      pool.alloc_bytes(integral_job_bytes(std::max<size_t>(ireq.size(), 1))),
+                                      pool.alloc_bytes(solid_job_bytes(ireq.size())), ctx.upload, st);
         ctx.upload.upload(scenes + k0, sd.data() + k0, (k1 - k0) * sizeof(SceneDev), st);
         launch_mark_root_cells(scenes, int32_t(k0), int32_t(k1 - k0), st);
         std::vector<int32_t> order;
@@ -1099,7 +1146,28 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
     launch_prefix_extract(bitmap, total_words, wsums, dev_word_begin, scenes, n, prefix, vertices, st);
 
     // ---- field (VH:827-888) ----
-    launch_field(vertices, uint32_t(nverts), scenes, values, st);
+    std::vector<BrickList> bricks; // lists of the steps at which some scene's bricks are kept
+    uint64_t brick_waves = 0;
+    if (by_bricks && nverts > 0)
+        for (int32_t i = 0; i < nlists; ++i)
+        {
+            const bool any = std::any_of(sd.begin(), sd.end(), [&](const SceneDev& d) {
+                return d.start + d.level - d.brick_shift == i;
+            });
+            if (!any || ctx.level_sizes[i] == 0)
+                continue;
+            bricks.push_back(BrickList{ ctx.level_lists[i], ctx.level_sizes[i], i, brick_waves });
+            brick_waves += ctx.level_sizes[i];
+        }
+    if (!bricks.empty())
+    {
+        BrickList* lists = pool.alloc<BrickList>(bricks.size());
+        ctx.upload.upload(lists, bricks.data(), bricks.size() * sizeof(BrickList), st);
+        launch_mark_bricks(lists, int32_t(bricks.size()), brick_waves, scenes, st);
+        launch_field_bricks(lists, int32_t(bricks.size()), brick_waves, scenes, bitmap, prefix, values, st);
+    }
+    else
+        launch_field(vertices, uint32_t(nverts), scenes, values, st);
     ctx.vertices = vertices;
     ctx.values = values;
 

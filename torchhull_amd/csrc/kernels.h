@@ -25,9 +25,22 @@ struct IntegralRequest
     int32_t dtype;
     int64_t B, H, W;
     float* padded;
+    // solid maps (common.h), built with the integral images where `solid` is not null: the maps and the cameras'
+    // bounds, and scratch of solid_scratch_bytes(B, H, W) bytes
+    uint8_t* solid;
+    CullCamera* cull;
+    void* solid_scratch;
+    const float* transforms;
+    int32_t opengl;
+    float corner[3];
+    float length;
 };
-void launch_integral_images_padded(const IntegralRequest* req, int32_t n, float* carry, void* job_buf, Uploader& up,
-                                   hipStream_t st);
+uint64_t solid_map_bytes(int64_t B, int64_t H, int64_t W);
+uint64_t solid_scratch_bytes(int64_t B, int64_t H, int64_t W);
+size_t solid_job_bytes(size_t njobs);
+// `solid_jobs`: solid_job_bytes(n) bytes of device scratch, unused without solid maps.
+void launch_integral_images_padded(const IntegralRequest* req, int32_t n, float* carry, void* job_buf,
+                                   void* solid_jobs, Uploader& up, hipStream_t st);
 
 // ---- octree carving (vh_kernels.hip) ----
 constexpr int kCarveThreads = 256;
@@ -83,6 +96,22 @@ void launch_prefix_extract(const uint32_t* bitmap, uint64_t nwords, const uint32
 // Self-test: div2_shared against the IEEE division on `count` random operand
 // triples; adds the number of differing quotients to *mismatches.
 void launch_div2_check(uint64_t count, uint64_t seed, unsigned long long* mismatches, hipStream_t st);
+
+// One octree list that holds bricks: the cells kept up to a carving step.
+struct BrickList
+{
+    const uint64_t* keys;
+    uint32_t count;
+    int32_t step;
+    uint64_t begin; // first wavefront of this list
+};
+// Marks the bricks of the lists (scenes whose brick level is reached at the list's step) in their scenes' brick
+// bitmaps, which are zero.  `waves`: the summed counts of the lists.
+void launch_mark_bricks(const BrickList* lists, int32_t nlists, uint64_t waves, const SceneDev* scenes,
+                        hipStream_t st);
+// Field values by bricks: as launch_field for all vertices of the lists' bricks, written at the vertices' ranks.
+void launch_field_bricks(const BrickList* lists, int32_t nlists, uint64_t waves, const SceneDev* scenes,
+                         const uint32_t* bitmap, const uint32_t* prefix, float* values, hipStream_t st);
 
 // Field value of every vertex: product over cameras of the bilinear mask sample.
 void launch_field(const uint64_t* vertices, uint32_t n, const SceneDev* scenes, float* values, hipStream_t st);
