@@ -322,6 +322,7 @@ struct SceneDev
     // field by bricks (null: not used): one bit per brick of 2^brick_shift cells per side of the scene's octree,
     // set for the bricks among the kept cells
     uint32_t* bricks;
+    uint8_t* group_flags; // with bricks: flags of the groups of 4 words of the vertex bitmap (group_flags_kernel)
     int32_t brick_shift;
     int32_t pad_;
 };

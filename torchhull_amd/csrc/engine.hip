@@ -670,7 +670,7 @@ make_plan(Context& ctx, std::vector<int64_t> sig, const std::vector<uint64_t>& r
         i_mask.push_back(add(p->cap[i]));
         i_bc.push_back(add(size_t(nb) * sizeof(uint32_t)));
         i_bo.push_back(add(size_t(nb) * sizeof(uint32_t)));
-        i_sums.push_back(add((size_t(scan_blocks(nb)) + 1) * sizeof(uint32_t)));
+        i_sums.push_back(add(size_t(scan_sums_room(nb)) * sizeof(uint32_t)));
     }
     size_t total = 0;
     std::vector<size_t> off(sizes.size());
@@ -815,6 +815,7 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
     // expensive cells and ends with the cheapest ones instead of finishing on a tail of many-camera
     // cells.  Each scene's own cells keep the reference's parent-major order, so no result depends on it.
     const bool by_bricks = solid_maps_pay(in, n0);
+    uint64_t most_flags = 0;
     auto add_scenes = [&](size_t k0, int32_t start) {
         const size_t k1 = all.size();
         std::vector<IntegralRequest> ireq;
@@ -845,11 +846,13 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
             d.start = start;
             const uint64_t R = uint64_t(1) << sc.level, R1 = R + 1;
             d.row_words = uint32_t((R1 + 31) / 32);
+            if (by_bricks)
+                d.row_words = (d.row_words + 3u) & ~3u; // whole groups of words (launch_dilate_groups)
             d.bitmap_offset = total_words;
             d.cell_row_words = uint32_t((R + 31) / 32);
             word_begin.push_back(total_words);
             total_words += R1 * R1 * d.row_words;
-            cell_words += R * R * d.cell_row_words;
+            cell_words += (R * R * d.cell_row_words + 3) & ~uint64_t(3); // 16-byte aligned scenes
             last_step = std::max(last_step, start + d.level);
             if (d.B > 0)
             {
@@ -881,6 +884,9 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
         {
             sd[s].brick_shift = std::min(kBrickShift, sd[s].level);
             brick_words += ((uint64_t(1) << (3 * (sd[s].level - sd[s].brick_shift))) + 31) / 32;
+            const uint64_t flags = group_flag_bytes(sd[s].level, sd[s].brick_shift, sd[s].row_words);
+            sd[s].group_flags = pool.alloc<uint8_t>(flags);
+            most_flags = std::max(most_flags, flags);
         }
         uint32_t* cells = pool.alloc<uint32_t>(std::max<uint64_t>(cell_words + brick_words, 1));
         launch_fill_u32(cells, cell_words + brick_words, 0u, st);
@@ -898,7 +904,7 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
         for (size_t s = k0; s < k1; ++s)
         {
             sd[s].cells = cells + off;
-            off += (uint64_t(1) << (2 * sd[s].level)) * sd[s].cell_row_words;
+            off += ((uint64_t(1) << (2 * sd[s].level)) * sd[s].cell_row_words + 3) & ~uint64_t(3);
         }
         uint64_t carry_floats = 0;
         for (const auto& r : ireq)
@@ -1070,7 +1076,7 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
         uint8_t* mask = pool.alloc<uint8_t>(count);
         uint32_t* bcount = pool.alloc<uint32_t>(nb);
         uint32_t* boff = pool.alloc<uint32_t>(nb);
-        uint32_t* sums = pool.alloc<uint32_t>(scan_blocks(nb) + 1);
+        uint32_t* sums = pool.alloc<uint32_t>(scan_sums_room(nb));
         if (ctx.profile)
             THULL_HIP(hipEventRecord(ctx.event(2 * i), st));
         const int32_t split = launch_carve_classify(list, count, i, scenes, mask, bcount, dev_tests + i, ctx.tuning, st);
@@ -1127,10 +1133,36 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
     ctx.upload.upload(dev_word_begin, word_begin.data(), (n + 1) * sizeof(uint64_t), st);
     uint32_t* bitmap = pool.alloc<uint32_t>(std::max<uint64_t>(total_words, 1));
     uint32_t* prefix = pool.alloc<uint32_t>(std::max<uint64_t>(total_words, 1));
+    std::vector<BrickList> bricks; // lists of the steps at which some scene's bricks are kept
+    uint64_t brick_waves = 0;
+    if (by_bricks)
+        for (int32_t i = 0; i < nlists; ++i)
+        {
+            const bool any = std::any_of(sd.begin(), sd.end(), [&](const SceneDev& d) {
+                return d.start + d.level - d.brick_shift == i;
+            });
+            if (!any || ctx.level_sizes[i] == 0)
+                continue;
+            bricks.push_back(BrickList{ ctx.level_lists[i], ctx.level_sizes[i], i, brick_waves });
+            brick_waves += ctx.level_sizes[i];
+        }
+    BrickList* brick_lists = nullptr;
+    if (!bricks.empty())
+    {
+        brick_lists = pool.alloc<BrickList>(bricks.size());
+        ctx.upload.upload(brick_lists, bricks.data(), bricks.size() * sizeof(BrickList), st);
+        launch_mark_bricks(brick_lists, int32_t(bricks.size()), brick_waves, scenes, st);
+    }
+    if (by_bricks)
+        launch_group_flags(scenes, n, most_flags, st);
     // dilation + tile popcount sums, scan of the sums, then word prefixes + vertex keys
     const uint32_t wblocks = scan_blocks(total_words);
-    uint32_t* wsums = pool.alloc<uint32_t>(wblocks + 1);
-    launch_dilate_cells(bitmap, total_words, dev_word_begin, scenes, n, wsums, st);
+    uint32_t* wsums = pool.alloc<uint32_t>(scan_sums_room(total_words));
+    uint64_t* filled = by_bricks ? pool.alloc<uint64_t>(filled_words(total_words)) : nullptr;
+    if (by_bricks)
+        launch_dilate_groups(bitmap, total_words, dev_word_begin, scenes, n, wsums, filled, st);
+    else
+        launch_dilate_cells(bitmap, total_words, dev_word_begin, scenes, n, wsums, st);
     uint64_t nverts = 0;
     if (wblocks > 0)
     {
@@ -1143,29 +1175,15 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
     check_u32(nverts, "sparse field size");
     uint64_t* vertices = pool.alloc<uint64_t>(std::max<uint64_t>(nverts, 1));
     float* values = pool.alloc<float>(std::max<uint64_t>(nverts, 1));
-    launch_prefix_extract(bitmap, total_words, wsums, dev_word_begin, scenes, n, prefix, vertices, st);
+    if (by_bricks)
+        launch_extract_groups(bitmap, total_words, filled, wsums, dev_word_begin, scenes, n, prefix, vertices, st);
+    else
+        launch_prefix_extract(bitmap, total_words, wsums, dev_word_begin, scenes, n, prefix, vertices, st);
 
     // ---- field (VH:827-888) ----
-    std::vector<BrickList> bricks; // lists of the steps at which some scene's bricks are kept
-    uint64_t brick_waves = 0;
-    if (by_bricks && nverts > 0)
-        for (int32_t i = 0; i < nlists; ++i)
-        {
-            const bool any = std::any_of(sd.begin(), sd.end(), [&](const SceneDev& d) {
-                return d.start + d.level - d.brick_shift == i;
-            });
-            if (!any || ctx.level_sizes[i] == 0)
-                continue;
-            bricks.push_back(BrickList{ ctx.level_lists[i], ctx.level_sizes[i], i, brick_waves });
-            brick_waves += ctx.level_sizes[i];
-        }
-    if (!bricks.empty())
-    {
-        BrickList* lists = pool.alloc<BrickList>(bricks.size());
-        ctx.upload.upload(lists, bricks.data(), bricks.size() * sizeof(BrickList), st);
-        launch_mark_bricks(lists, int32_t(bricks.size()), brick_waves, scenes, st);
-        launch_field_bricks(lists, int32_t(bricks.size()), brick_waves, scenes, bitmap, prefix, values, st);
-    }
+    if (by_bricks)
+        launch_field_bricks(brick_lists, int32_t(bricks.size()), nverts > 0 ? brick_waves : 0, scenes, bitmap, prefix,
+                            values, st);
     else
         launch_field(vertices, uint32_t(nverts), scenes, values, st);
     ctx.vertices = vertices;
@@ -1210,7 +1228,7 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
         uint32_t* info = pool.alloc<uint32_t>(nverts);
         uint32_t* ntv = pool.alloc<uint32_t>(nverts);
         uint32_t* tbase = pool.alloc<uint32_t>(nverts);
-        uint32_t* sums = pool.alloc<uint32_t>(scan_blocks(nverts) + 1);
+        uint32_t* sums = pool.alloc<uint32_t>(scan_sums_room(nverts));
         uint32_t* emask = nullptr;
         uint32_t* vbase = nullptr;
         launch_mc_classify(plan, info, ntv, st);
@@ -1663,7 +1681,7 @@ mc_run_common(Context& c, thull::McPlan plan, McGridUpload* dgrid, bool unique, 
     uint32_t* info = pool.alloc<uint32_t>(n);
     uint32_t* ntv = pool.alloc<uint32_t>(n);
     uint32_t* tbase = pool.alloc<uint32_t>(n);
-    uint32_t* sums = pool.alloc<uint32_t>(scan_blocks(n) + 1);
+    uint32_t* sums = pool.alloc<uint32_t>(scan_sums_room(n));
     uint32_t* emask = nullptr;
     uint32_t* vbase = nullptr;
     // the last scan sends the totals to the host (compact meshes: the output vertices, with the triangle
@@ -1837,7 +1855,7 @@ thull_marching_cubes_sparse_run(thull_ctx* ctx,
             launch_fill_u32(reinterpret_cast<uint32_t*>(dev_total), 4, 0u, st);
             launch_fill_u32(bitmap, nwords, 0u, st);
             launch_mark_coo(indices, uint64_t(nnz), dgrid, bitmap, dev_total + 1, st);
-            uint32_t* sums = pool.alloc<uint32_t>(scan_blocks(nwords) + 1);
+            uint32_t* sums = pool.alloc<uint32_t>(scan_sums_room(nwords));
             // the scan sends the number of set bits (at most nnz) and the flag to the host; the vertex list
             // goes out before the host learns them
             const ScanNotify note = c.notify.next(dev_total + 1);

@@ -109,6 +109,19 @@ struct BrickList
 // bitmaps, which are zero.  `waves`: the summed counts of the lists.
 void launch_mark_bricks(const BrickList* lists, int32_t nlists, uint64_t waves, const SceneDev* scenes,
                         hipStream_t st);
+// Flags of the groups of 4 words of the scenes' vertex bitmaps that marked bricks reach, group_flag_bytes per scene
+// (`most`: the largest scene's).
+uint64_t group_flag_bytes(int32_t level, int32_t brick_shift, uint32_t row_words);
+void launch_group_flags(const SceneDev* scenes, int32_t nscenes, uint64_t most, hipStream_t st);
+// launch_dilate_cells and launch_prefix_extract for scenes whose group flags are set: rows of whole groups of 4 words,
+// every scene's words a multiple of 4, and prefixes only of groups with vertices and of every scene's first group.
+// `filled`: filled_words(nwords) words of bits of those groups, from the first launch to the second.
+uint64_t filled_words(uint64_t nwords);
+void launch_dilate_groups(uint32_t* verts, uint64_t nwords, const uint64_t* scene_word_begin, const SceneDev* scenes,
+                          int32_t nscenes, uint32_t* block_sums, uint64_t* filled, hipStream_t st);
+void launch_extract_groups(const uint32_t* bitmap, uint64_t nwords, const uint64_t* filled,
+                           const uint32_t* block_offsets, const uint64_t* scene_word_begin, const SceneDev* scenes,
+                           int32_t nscenes, uint32_t* prefix, uint64_t* vertices, hipStream_t st);
 // Field values by bricks: as launch_field for all vertices of the lists' bricks, written at the vertices' ranks.
 void launch_field_bricks(const BrickList* lists, int32_t nlists, uint64_t waves, const SceneDev* scenes,
                          const uint32_t* bitmap, const uint32_t* prefix, float* values, hipStream_t st);

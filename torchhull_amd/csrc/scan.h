@@ -107,19 +107,36 @@ struct ScanGuard
     uint32_t* overflow = nullptr;
 };
 
-// Single-block exclusive scan of the block sums; writes the grand total (64-bit).
+// Group k of 4 sums with the entries past n as zeros.
+__device__ __forceinline__ uint4
+load_sums4(const uint4* v, uint32_t k, uint32_t n)
+{
+    uint4 u = v[k];
+    u.y = 4 * k + 1 < n ? u.y : 0u;
+    u.z = 4 * k + 2 < n ? u.z : 0u;
+    u.w = 4 * k + 3 < n ? u.w : 0u;
+    return u;
+}
+
+// Single-block exclusive scan of the block sums (16-byte aligned, room for nblocks rounded up to 4); writes the grand
+// total (64-bit).  A thread takes a run of whole 16-byte groups (the three scans of a level-11 hull, the largest of
+// 70 000 sums: 167 -> 39 us).
 template <typename Tag = void>
 __global__ __launch_bounds__(1024) void
 scan_block_sums_kernel(uint32_t* sums, uint32_t nblocks, unsigned long long* total_out, ScanNotify note = {},
                        ScanGuard guard = {})
 {
     __shared__ unsigned long long lds[1024 / 64];
-    const uint32_t per = (nblocks + 1023) / 1024;
-    const uint32_t begin = threadIdx.x * per;
+    const uint32_t groups = (nblocks + 3) / 4, per = (groups + 1023) / 1024;
+    const uint32_t begin = threadIdx.x * per, end = min(begin + per, groups);
+    uint4* const v = reinterpret_cast<uint4*>(sums);
     unsigned long long local = 0;
-    for (uint32_t k = 0; k < per; ++k)
-        if (begin + k < nblocks)
-            local += sums[begin + k];
+#pragma unroll 4
+    for (uint32_t k = begin; k < end; ++k)
+    {
+        const uint4 u = load_sums4(v, k, nblocks);
+        local += (unsigned long long)u.x + u.y + u.z + u.w;
+    }
     // block scan of 64-bit partial sums
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     unsigned long long inc = local;
@@ -139,28 +156,30 @@ scan_block_sums_kernel(uint32_t* sums, uint32_t nblocks, unsigned long long* tot
             off += lds[w];
         total += lds[w];
     }
-    unsigned long long run = off + inc - local;
-    for (uint32_t k = 0; k < per; ++k)
-        if (begin + k < nblocks)
-        {
-            uint32_t v = sums[begin + k];
-            sums[begin + k] = uint32_t(run);
-            run += v;
-        }
     if (threadIdx.x == 0)
     {
-        if (guard.overflow != nullptr && total > guard.cap)
+        unsigned long long t = total;
+        if (guard.overflow != nullptr && t > guard.cap)
         {
             *guard.overflow = 1u;
-            total = guard.cap;
+            t = guard.cap;
         }
-        *total_out = total;
+        *total_out = t;
         if (note.slot != nullptr)
         {
-            note.slot[0] = total;
+            note.slot[0] = t;
             note.slot[1] = note.extra != nullptr ? *note.extra : 0ull;
             __hip_atomic_store(note.slot + 2, note.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
         }
+    }
+    unsigned long long run = off + inc - local;
+#pragma unroll 4
+    for (uint32_t k = begin; k < end; ++k)
+    {
+        const uint4 u = load_sums4(v, k, nblocks);
+        v[k] = make_uint4(uint32_t(run), uint32_t(run + u.x), uint32_t(run + u.x + u.y),
+                          uint32_t(run + u.x + u.y + u.z));
+        run += (unsigned long long)u.x + u.y + u.z + u.w;
     }
 }
 
@@ -174,20 +193,12 @@ scan_block_sums2_kernel(uint32_t* a, uint32_t* b, uint32_t n, unsigned long long
     const uint32_t groups = (n + 3) / 4, per = (groups + 1023) / 1024;
     const uint32_t begin = threadIdx.x * per, end = min(begin + per, groups);
     uint4* const v[2] = { reinterpret_cast<uint4*>(a), reinterpret_cast<uint4*>(b) };
-    // group k with the entries past n as zeros
-    const auto load = [&](int q, uint32_t k) {
-        uint4 u = v[q][k];
-        u.y = 4 * k + 1 < n ? u.y : 0u;
-        u.z = 4 * k + 2 < n ? u.z : 0u;
-        u.w = 4 * k + 3 < n ? u.w : 0u;
-        return u;
-    };
     unsigned long long sum[2] = { 0, 0 };
     for (uint32_t k = begin; k < end; ++k)
 #pragma unroll
         for (int q = 0; q < 2; ++q)
         {
-            const uint4 u = load(q, k);
+            const uint4 u = load_sums4(v[q], k, n);
             sum[q] += (unsigned long long)u.x + u.y + u.z + u.w;
         }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -231,7 +242,7 @@ scan_block_sums2_kernel(uint32_t* a, uint32_t* b, uint32_t n, unsigned long long
 #pragma unroll
         for (int q = 0; q < 2; ++q)
         {
-            const uint4 u = load(q, k);
+            const uint4 u = load_sums4(v[q], k, n);
             const unsigned long long r = run[q];
             v[q][k] = make_uint4(uint32_t(r), uint32_t(r + u.x), uint32_t(r + u.x + u.y),
                                  uint32_t(r + u.x + u.y + u.z));
@@ -359,11 +370,18 @@ scan_small_kernel(L load, uint32_t n, uint32_t* out, unsigned long long* total_o
 }
 
 // Exclusive scan of load(i), i in [0, n), into out[0, n).  `block_sums` must
-// hold scan_blocks(n) entries; the 64-bit total lands in *total_dev.
+// hold scan_sums_room(n) entries, 16-byte aligned; the 64-bit total lands in *total_dev.
 inline uint32_t
 scan_blocks(uint64_t n)
 {
     return uint32_t((n + kScanTile - 1) / kScanTile);
+}
+
+// Entries of an array of block sums: at least one group of 4, whole groups.
+inline uint32_t
+scan_sums_room(uint64_t n)
+{
+    return std::max((scan_blocks(n) + 3u) & ~3u, 4u);
 }
 
 // `note` (optional, n > 0) also sends the total to the host; `guard` (optional) clamps it.  Every
