@@ -1073,25 +1073,31 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
         THULL_CHECK(i < kMaxSteps, "too many carving steps");
         const int32_t room = capacity - int32_t(all.size()); // roots that may join at the next boundary
         const uint32_t nb = blocks_for(count, kCarveThreads);
+        const bool compact = count <= kCompactParents;
         uint8_t* mask = pool.alloc<uint8_t>(count);
         uint32_t* bcount = pool.alloc<uint32_t>(nb);
         uint32_t* boff = pool.alloc<uint32_t>(nb);
         uint32_t* sums = pool.alloc<uint32_t>(scan_sums_room(nb));
         if (ctx.profile)
             THULL_HIP(hipEventRecord(ctx.event(2 * i), st));
-        const int32_t split = launch_carve_classify(list, count, i, scenes, mask, bcount, dev_tests + i, ctx.tuning, st);
+        const int32_t split = launch_carve_classify(list, count, i, scenes, mask, bcount, dev_tests + i, ctx.tuning,
+                                                    st, nullptr, 0, nullptr, !compact);
         if (ctx.profile)
             THULL_HIP(hipEventRecord(ctx.event(2 * i + 1), st));
         // the scan sends the next level's size (and the camera tests) to the host; the children go out
         // before the host learns their number (8 per parent at most), so the scatter runs while the host
         // queues the next level
         const ScanNotify note = ctx.notify.next(dev_tests + i);
-        exclusive_scan(LoadU32{ bcount }, nb, boff, sums, dev_total, st, note);
+        if (!compact)
+            exclusive_scan(LoadU32{ bcount }, nb, boff, sums, dev_total, st, note);
         uint64_t* children = pool.alloc<uint64_t>(std::max<uint64_t>(uint64_t(count) * 8 + uint64_t(room), 1));
         bool target = false; // a scene ends at step i + 1
         for (const SceneDev& d : sd)
             target |= d.start + d.level == i + 1;
-        launch_carve_scatter(list, count, mask, boff, children, i + 1, scenes, target, st);
+        if (compact)
+            launch_carve_compact(list, count, mask, children, i + 1, scenes, target, dev_total, note, st);
+        else
+            launch_carve_scatter(list, count, mask, boff, children, i + 1, scenes, target, st);
         unsigned long long got[2];
         if (!ctx.notify.wait(note, st, got))
         {

@@ -64,7 +64,7 @@ int32_t carve_split_factor(uint32_t n, const CarveTuning& tune);
 int32_t launch_carve_classify(const uint64_t* parents, uint32_t n, int32_t step, const SceneDev* scenes,
                               uint8_t* child_mask, uint32_t* block_counts, unsigned long long* tests,
                               const CarveTuning& tune, hipStream_t st, const unsigned long long* dev_n = nullptr,
-                              int32_t split_hint = 0, uint32_t* cursors = nullptr);
+                              int32_t split_hint = 0, uint32_t* cursors = nullptr, bool counts = true);
 
 // Writes the occupied children of every parent, parent-major and child-minor,
 // at `block_offsets[block]` + the in-block prefix.  With `mark_leaves`, the
@@ -75,6 +75,13 @@ void launch_carve_scatter(const uint64_t* parents, uint32_t n, const uint8_t* ch
                           const uint32_t* block_offsets, uint64_t* children, int32_t child_step,
                           const SceneDev* scenes, bool mark_leaves, hipStream_t st,
                           const unsigned long long* dev_n = nullptr, uint64_t out_cap = ~uint64_t(0));
+// Block counts, their scan and launch_carve_scatter of a level of at most kCompactParents parents in one launch
+// (masks 16-byte aligned); total and note as in exclusive_scan.
+struct ScanNotify;
+constexpr uint32_t kCompactParents = 1u << 17;
+void launch_carve_compact(const uint64_t* parents, uint32_t n, const uint8_t* child_mask, uint64_t* children,
+                          int32_t child_step, const SceneDev* scenes, bool mark_leaves, unsigned long long* total,
+                          const ScanNotify& note, hipStream_t st);
 // Sets the root cell of every level-0 scene among scenes first .. first + nscenes - 1.
 void launch_mark_root_cells(const SceneDev* scenes, int32_t first, int32_t nscenes, hipStream_t st);
 // Vertex bitmap (all words, no clearing needed) = leaf cells dilated by {0,1}^3.

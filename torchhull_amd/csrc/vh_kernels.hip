@@ -1679,6 +1679,12 @@ carve_classify_split_kernel(const uint64_t* __restrict__ parents,
         atomicAdd(tests_out, (unsigned long long)tsum);
 }
 
+__device__ __forceinline__ uint32_t
+popc4(const uint4& v)
+{
+    return uint32_t(__popc(v.x) + __popc(v.y) + __popc(v.z) + __popc(v.w));
+}
+
 __global__ __launch_bounds__(kCarveThreads) void
 carve_count_kernel(const uint8_t* __restrict__ child_mask, uint32_t n, uint32_t* __restrict__ block_counts,
                    const unsigned long long* __restrict__ dev_n) // optional: n = min(n, *dev_n)
@@ -1758,6 +1764,31 @@ mark_leaf_children_wave(const SceneDev* __restrict__ scenes, int32_t child_step,
     }
 }
 
+// The kept children of a block's parents, one contiguous range of the list from `first`: assembled in LDS at `off` and
+// written with coalesced stores.  All threads of the block call this.
+__device__ __forceinline__ void
+write_children(uint64_t* stage, uint64_t key, uint32_t mask, uint32_t off, uint32_t total, uint64_t first,
+               uint64_t* __restrict__ children, uint64_t out_cap, int32_t child_step,
+               const SceneDev* __restrict__ scenes, bool mark_leaves)
+{
+    if (mask != 0u)
+    {
+        const uint32_t s = key_scene(key), x = 2 * key_x(key), y = 2 * key_y(key), z = 2 * key_z(key);
+        // VH:694-711: children of a parent in child order (x bit, y bit, z bit)
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+            if (mask & (1u << c))
+                stage[off++] = pack_key(s, x + (c & 1), y + ((c >> 1) & 1), z + ((c >> 2) & 1));
+    }
+    __syncthreads();
+    uint64_t* dst = children + first;
+    for (uint32_t q = threadIdx.x; q < total; q += kCarveThreads)
+        if (first + q < out_cap)
+            dst[q] = stage[q];
+    if (mark_leaves)
+        mark_leaf_children_wave(scenes, child_step, key, mask);
+}
+
 __global__ __launch_bounds__(kCarveThreads) void
 carve_scatter_kernel(const uint64_t* __restrict__ parents,
                      uint32_t n,
@@ -1770,8 +1801,6 @@ carve_scatter_kernel(const uint64_t* __restrict__ parents,
                      const unsigned long long* __restrict__ dev_n, // optional: n = min(n, *dev_n)
                      uint64_t out_cap)                             // children past this index are dropped
 {
-    // the block's children are one contiguous range of the list: they are assembled in LDS and
-    // written with coalesced stores
     __shared__ uint32_t lds[kCarveThreads / 64];
     __shared__ uint64_t stage[kCarveThreads * 8];
     if (dev_n != nullptr)
@@ -1780,24 +1809,47 @@ carve_scatter_kernel(const uint64_t* __restrict__ parents,
     const uint32_t mask = (t < n) ? child_mask[t] : 0u;
     const uint64_t key = (t < n) ? parents[t] : 0; // read with the mask, ahead of the block sum
     uint32_t total;
-    uint32_t off = block_exclusive_sum(__popc(mask), lds, total);
-    if (mask != 0u)
+    const uint32_t off = block_exclusive_sum(__popc(mask), lds, total);
+    write_children(stage, key, mask, off, total, block_offsets[blockIdx.x], children, out_cap, child_step, scenes,
+                   mark_leaves);
+}
+
+// Count, scan and scatter of a level of at most kCompactParents in one launch: every block sums the masks of all
+// parents before its own (a byte each, a few 16-byte loads per thread from L2), so no block waits for another, and
+// the last one has the total for the host.  Small levels spend their time in launches: a level-7 hull of 8 cameras
+// 420 -> 384 us, a level-8 one of 16 540 -> 487.  At kCompactParents a thread reads 32 groups of masks at most.
+__global__ __launch_bounds__(kCarveThreads) void
+carve_compact_kernel(const uint64_t* __restrict__ parents, uint32_t n, const uint8_t* __restrict__ child_mask,
+                     uint64_t* __restrict__ children, int32_t child_step, const SceneDev* __restrict__ scenes,
+                     bool mark_leaves, unsigned long long* __restrict__ total_out, ScanNotify note)
+{
+    __shared__ uint32_t lds[kCarveThreads / 64];
+    __shared__ uint64_t stage[kCarveThreads * 8];
+    const uint32_t t = blockIdx.x * kCarveThreads + threadIdx.x;
+    const uint32_t mask = (t < n) ? child_mask[t] : 0u;
+    const uint64_t key = (t < n) ? parents[t] : 0;
+    uint32_t before = 0u;
+#pragma unroll 4
+    for (uint32_t g = threadIdx.x; g < blockIdx.x * (kCarveThreads / 16u); g += kCarveThreads)
+        before += popc4(reinterpret_cast<const uint4*>(child_mask)[g]);
+    // one block sum of both: at most 8 children of 256 parents in the low 12 bits, the sum before above
+    static_assert(uint64_t(kCompactParents) * 8u <= uint64_t(1) << 20, "sums fit 20 bits");
+    uint32_t both;
+    const uint32_t mine = block_exclusive_sum((before << 12) | __popc(mask), lds, both);
+    const uint32_t first = both >> 12, total = both & 4095u;
+    if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0)
     {
-        const uint32_t s = key_scene(key), x = 2 * key_x(key), y = 2 * key_y(key), z = 2 * key_z(key);
-        // VH:694-711: children of a parent in child order (x bit, y bit, z bit)
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-            if (mask & (1u << c))
-                stage[off++] = pack_key(s, x + (c & 1), y + ((c >> 1) & 1), z + ((c >> 2) & 1));
+        const unsigned long long all = first + total;
+        *total_out = all;
+        if (note.slot != nullptr)
+        {
+            note.slot[0] = all;
+            note.slot[1] = note.extra != nullptr ? *note.extra : 0ull;
+            __hip_atomic_store(note.slot + 2, note.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
     }
-    __syncthreads();
-    const uint64_t first = block_offsets[blockIdx.x];
-    uint64_t* dst = children + first;
-    for (uint32_t q = threadIdx.x; q < total; q += kCarveThreads)
-        if (first + q < out_cap)
-            dst[q] = stage[q];
-    if (mark_leaves)
-        mark_leaf_children_wave(scenes, child_step, key, mask);
+    write_children(stage, key, mask, mine & 4095u, total, first, children, ~uint64_t(0), child_step, scenes,
+                   mark_leaves);
 }
 
 int32_t
@@ -1812,12 +1864,17 @@ launch_carve_classify(const uint64_t* parents,
                       hipStream_t st,
                       const unsigned long long* dev_n,
                       int32_t split_hint,
-                      uint32_t* cursors)
+                      uint32_t* cursors,
+                      bool counts)
 {
     if (n == 0)
         return 0;
     const int32_t split = dev_n != nullptr ? split_hint : carve_split_factor(n, tune);
     const uint64_t nb = blocks_for(n, kCarveThreads);
+    const auto count = [&] {
+        if (counts)
+            carve_count_kernel<<<nb, kCarveThreads, 0, st>>>(child_mask, n, block_counts, dev_n);
+    };
     if (dev_n != nullptr && split == 1)
     {
         // persistent workgroups: as many as the CUs hold at the kernel's occupancy (3 per CU), a multiple
@@ -1833,28 +1890,28 @@ launch_carve_classify(const uint64_t* parents,
         carve_classify_split_kernel<64><<<blocks_for(int64_t(n) * 64, 256), 256, 0, st>>>(parents, n, level_i, scenes,
                                                                                           child_mask, tests, dev_n);
         THULL_LAUNCH_CHECK();
-        carve_count_kernel<<<nb, kCarveThreads, 0, st>>>(child_mask, n, block_counts, dev_n);
+        count();
     }
     else if (split == 16)
     {
         carve_classify_split_kernel<16><<<blocks_for(int64_t(n) * 16, 256), 256, 0, st>>>(parents, n, level_i, scenes,
                                                                                           child_mask, tests, dev_n);
         THULL_LAUNCH_CHECK();
-        carve_count_kernel<<<nb, kCarveThreads, 0, st>>>(child_mask, n, block_counts, dev_n);
+        count();
     }
     else if (split == 4)
     {
         carve_classify_split_kernel<4><<<blocks_for(int64_t(n) * 4, 256), 256, 0, st>>>(parents, n, level_i, scenes,
                                                                                         child_mask, tests, dev_n);
         THULL_LAUNCH_CHECK();
-        carve_count_kernel<<<nb, kCarveThreads, 0, st>>>(child_mask, n, block_counts, dev_n);
+        count();
     }
     else if (split == 2)
     {
         carve_classify_split_kernel<2><<<blocks_for(int64_t(n) * 2, 256), 256, 0, st>>>(parents, n, level_i, scenes,
                                                                                         child_mask, tests, dev_n);
         THULL_LAUNCH_CHECK();
-        carve_count_kernel<<<nb, kCarveThreads, 0, st>>>(child_mask, n, block_counts, dev_n);
+        count();
     }
     else
     {
@@ -1902,6 +1959,17 @@ launch_carve_scatter(const uint64_t* parents,
         return;
     carve_scatter_kernel<<<blocks_for(n, kCarveThreads), kCarveThreads, 0, st>>>(
             parents, n, child_mask, block_offsets, children, child_step, scenes, mark_leaves, dev_n, out_cap);
+    THULL_LAUNCH_CHECK();
+}
+
+void
+launch_carve_compact(const uint64_t* parents, uint32_t n, const uint8_t* child_mask, uint64_t* children,
+                     int32_t child_step, const SceneDev* scenes, bool mark_leaves, unsigned long long* total,
+                     const ScanNotify& note, hipStream_t st)
+{
+    THULL_CHECK(n > 0 && n <= kCompactParents, "level size of a one-launch compaction");
+    carve_compact_kernel<<<blocks_for(n, kCarveThreads), kCarveThreads, 0, st>>>(
+            parents, n, child_mask, children, child_step, scenes, mark_leaves, total, note);
     THULL_LAUNCH_CHECK();
 }
 
@@ -2413,12 +2481,6 @@ dilate_group(const SceneDev& s, const WordGroup& q)
             out[k] |= c[k + 1] | (c[k + 1] << 1) | (c[k] >> 31);
     }
     return make_uint4(out[0], out[1], out[2], out[3]);
-}
-
-__device__ __forceinline__ uint32_t
-popc4(const uint4& v)
-{
-    return uint32_t(__popc(v.x) + __popc(v.y) + __popc(v.z) + __popc(v.w));
 }
 
 constexpr int kTileGroups = kScanTile / 4;
