@@ -705,6 +705,16 @@ make_plan(Context& ctx, std::vector<int64_t> sig, const std::vector<uint64_t>& r
     return ctx.plans.back().get();
 }
 
+// The most cameras of a scene (launch_carve_classify).
+static int32_t
+max_cameras(const std::vector<SceneDev>& sd)
+{
+    int32_t most = 0;
+    for (const SceneDev& d : sd)
+        most = std::max(most, d.B);
+    return most;
+}
+
 // The launches of a plan's carving loop, as captured into its graph: counters cleared by kernels (no
 // memset nodes), then per step the classification (a persistent work-queue kernel, or the lane-split
 // kernel on a capacity-sized grid), the scan of the block counts whose total is the next level's size,
@@ -730,8 +740,8 @@ record_plan(Context& ctx, const CarvePlan& p, const std::vector<SceneDev>& sd, i
         const uint32_t nb = blocks_for(p.cap[i], kCarveThreads);
         if (timed)
             THULL_HIP(hipEventRecord(ctx.event(2 * i), st));
-        launch_carve_classify(p.lists[i], p.cap[i], i, p.scenes, p.masks[i], p.bcount[i], tests + i, ctx.tuning, st,
-                              counts + i, p.split[i], p.cursors + 8 * i);
+        launch_carve_classify(p.lists[i], p.cap[i], i, p.scenes, p.masks[i], p.bcount[i], tests + i, ctx.tuning,
+                              max_cameras(sd), st, counts + i, p.split[i], p.cursors + 8 * i);
         if (timed)
             THULL_HIP(hipEventRecord(ctx.event(2 * i + 1), st));
         // the next level's size, clamped to its list's capacity (overflow: the run is repeated)
@@ -1081,7 +1091,7 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
         if (ctx.profile)
             THULL_HIP(hipEventRecord(ctx.event(2 * i), st));
         const int32_t split = launch_carve_classify(list, count, i, scenes, mask, bcount, dev_tests + i, ctx.tuning,
-                                                    st, nullptr, 0, nullptr, !compact);
+                                                    max_cameras(sd), st, nullptr, 0, nullptr, !compact);
         if (ctx.profile)
             THULL_HIP(hipEventRecord(ctx.event(2 * i + 1), st));
         // the scan sends the next level's size (and the camera tests) to the host; the children go out

@@ -57,14 +57,15 @@ struct CarveTuning
     uint32_t max_parents[4] = { 16384u, 131072u, 1048576u, 1048576u }; // G = 64, 16, 4, 2 up to these sizes
 };
 int32_t carve_split_factor(uint32_t n, const CarveTuning& tune);
-// `step`: the carving step (a scene's octree level is step - its start).
+// `step`: the carving step (a scene's octree level is step - its start).  `max_cameras`: the most cameras of a scene.
 // Device-driven levels (dev_n non-null): the level holds min(*dev_n, n) parents, n being the list's
 // capacity; the lanes per parent are `split_hint`, and with one lane per parent a persistent queue
 // kernel runs (carve_classify_queue_kernel, `cursors`: 8 words, zero at start).
 int32_t launch_carve_classify(const uint64_t* parents, uint32_t n, int32_t step, const SceneDev* scenes,
                               uint8_t* child_mask, uint32_t* block_counts, unsigned long long* tests,
-                              const CarveTuning& tune, hipStream_t st, const unsigned long long* dev_n = nullptr,
-                              int32_t split_hint = 0, uint32_t* cursors = nullptr, bool counts = true);
+                              const CarveTuning& tune, int32_t max_cameras, hipStream_t st,
+                              const unsigned long long* dev_n = nullptr, int32_t split_hint = 0,
+                              uint32_t* cursors = nullptr, bool counts = true);
 
 // Writes the occupied children of every parent, parent-major and child-minor,
 // at `block_offsets[block]` + the in-block prefix.  With `mark_leaves`, the

@@ -1007,56 +1007,56 @@ pixel_box(const Box& q, float fW, float fH)
                      to_upper<GL>(q.maxy, fH) };
 }
 
-// Projects one z-slice (3 x 3 points) of a parent's lattice for one camera and
-// reduces it to the quotient boxes of its four 2 x 2 point groups, box a + 2b
-// for x offset a and y offset b.  The fused row products are shared along the
+// Projects one z-slice (N x N points, 3 x 3 of a parent's lattice or 2 x 2 of a
+// child's) for one camera and reduces it to the quotient boxes of its 2 x 2 point
+// groups, box a + (N - 1) b for x offset a and y offset b.  The fused row products are shared along the
 // lattice axes: fmaf(A2, z, A3) per slice, fmaf(A1, y, .) per row and
 // fmaf(A0, x, .) per point, the nested fmaf chain of VH:150-153.  The
 // quotients take the shared-reciprocal division, checked once for the whole
 // slice (carve_div_in_range; the largest magnitude propagates NaN, so a NaN
 // operand fails the check too); a slice that fails is projected again with
 // the IEEE division (rare: a lattice point on a camera's principal plane, or
-// non-finite input), and `nanpts` gets bit u + 3v for each point whose
+// non-finite input), and `nanpts` gets bit u + Nv for each point whose
 // quotients hold a NaN.  A slice that passes has finite quotients only.
-template <bool GL>
+template <bool GL, int N>
 __device__ __forceinline__ void
-lattice_slice(const CarveCamera& cam, const float (&wx)[3], const float (&wy)[3], float wz, Box (&win)[4],
-              uint32_t& nanpts)
+lattice_slice(const CarveCamera& cam, const float (&wx)[N], const float (&wy)[N], float wz,
+              Box (&win)[(N - 1) * (N - 1)], uint32_t& nanpts)
 {
     const float ax = fmaf(cam.x2, wz, cam.x3);
     const float ay = fmaf(cam.y2, wz, cam.y3);
     const float ad = fmaf(cam.d2, wz, cam.d3);
-    float ppx[3][3], ppy[3][3]; // [v][u] quotients
-    float hi[3], lo[3];
+    float ppx[N][N], ppy[N][N]; // [v][u] quotients
+    float hi = 0.0f, lo = 0.0f;
 #pragma unroll
-    for (int v = 0; v < 3; ++v)
+    for (int v = 0; v < N; ++v)
     {
         const float bx = fmaf(cam.x1, wy[v], ax);
         const float by = fmaf(cam.y1, wy[v], ay);
         const float bd = fmaf(cam.d1, wy[v], ad);
-        float h[3], l[3];
+        float h = 0.0f, l = 0.0f;
 #pragma unroll
-        for (int u = 0; u < 3; ++u)
+        for (int u = 0; u < N; ++u)
         {
             const float cx = fmaf(cam.x0, wx[u], bx);
             const float cy = fmaf(cam.y0, wx[u], by);
             const float cd = fmaf(cam.d0, wx[u], bd);
-            h[u] = max_abs3_nan(cx, cy, cd);
-            l[u] = fabsf(cd);
+            const float hu = max_abs3_nan(cx, cy, cd);
+            h = u == 0 ? hu : __builtin_elementwise_maximum(h, hu);
+            l = u == 0 ? fabsf(cd) : fminf(l, fabsf(cd));
             div2_unchecked(cx, cy, cd, ppx[v][u], ppy[v][u]); // cx / cd, cy / cd when in range
         }
-        hi[v] = __builtin_elementwise_maximum(__builtin_elementwise_maximum(h[0], h[1]), h[2]);
-        lo[v] = fminf(fminf(l[0], l[1]), l[2]);
+        hi = v == 0 ? h : __builtin_elementwise_maximum(hi, h);
+        lo = v == 0 ? l : fminf(lo, l);
     }
     nanpts = 0u;
-    const float hs = __builtin_elementwise_maximum(__builtin_elementwise_maximum(hi[0], hi[1]), hi[2]);
-    if (carve_div_in_range(hs, fminf(fminf(lo[0], lo[1]), lo[2])))
+    if (carve_div_in_range(hi, lo))
     {
         // every quotient is finite: the boxes take the single-instruction minimum / maximum
 #pragma unroll
-        for (int bb = 0; bb < 2; ++bb)
+        for (int bb = 0; bb + 1 < N; ++bb)
 #pragma unroll
-            for (int a = 0; a < 2; ++a)
+            for (int a = 0; a + 1 < N; ++a)
             {
                 const float mnx0 = min_nn(ppx[bb][a], ppx[bb][a + 1]);
                 const float mnx1 = min_nn(ppx[bb + 1][a], ppx[bb + 1][a + 1]);
@@ -1066,18 +1066,18 @@ lattice_slice(const CarveCamera& cam, const float (&wx)[3], const float (&wy)[3]
                 const float mxx1 = max_nn(ppx[bb + 1][a], ppx[bb + 1][a + 1]);
                 const float mxy0 = max_nn(ppy[bb][a], ppy[bb][a + 1]);
                 const float mxy1 = max_nn(ppy[bb + 1][a], ppy[bb + 1][a + 1]);
-                win[a + 2 * bb] = Box{ min_nn(mnx0, mnx1), min_nn(mny0, mny1), max_nn(mxx0, mxx1), max_nn(mxy0, mxy1) };
+                win[a + (N - 1) * bb] = Box{ min_nn(mnx0, mnx1), min_nn(mny0, mny1), max_nn(mxx0, mxx1), max_nn(mxy0, mxy1) };
             }
         return;
     }
 #pragma unroll
-    for (int v = 0; v < 3; ++v)
+    for (int v = 0; v < N; ++v)
     {
         const float bx = fmaf(cam.x1, wy[v], ax);
         const float by = fmaf(cam.y1, wy[v], ay);
         const float bd = fmaf(cam.d1, wy[v], ad);
 #pragma unroll
-        for (int u = 0; u < 3; ++u)
+        for (int u = 0; u < N; ++u)
         {
             const float cx = fmaf(cam.x0, wx[u], bx);
             const float cy = fmaf(cam.y0, wx[u], by);
@@ -1085,14 +1085,14 @@ lattice_slice(const CarveCamera& cam, const float (&wx)[3], const float (&wy)[3]
             ppx[v][u] = cx / cd;
             ppy[v][u] = cy / cd;
             if (ppx[v][u] != ppx[v][u] || ppy[v][u] != ppy[v][u])
-                nanpts |= 1u << (u + 3 * v);
+                nanpts |= 1u << (u + N * v);
         }
     }
     // NaN quotients are left out (fminf / fmaxf); an all-NaN group gets the box (+inf, -inf)
 #pragma unroll
-    for (int bb = 0; bb < 2; ++bb)
+    for (int bb = 0; bb + 1 < N; ++bb)
 #pragma unroll
-        for (int a = 0; a < 2; ++a)
+        for (int a = 0; a + 1 < N; ++a)
         {
             const float mnx0 = fminf(ppx[bb][a], ppx[bb][a + 1]);
             const float mnx1 = fminf(ppx[bb + 1][a], ppx[bb + 1][a + 1]);
@@ -1102,7 +1102,7 @@ lattice_slice(const CarveCamera& cam, const float (&wx)[3], const float (&wy)[3]
             const float mxx1 = fmaxf(ppx[bb + 1][a], ppx[bb + 1][a + 1]);
             const float mxy0 = fmaxf(ppy[bb][a], ppy[bb][a + 1]);
             const float mxy1 = fmaxf(ppy[bb + 1][a], ppy[bb + 1][a + 1]);
-            win[a + 2 * bb] = Box{ fminf(fminf(mnx0, mnx1), INFINITY), fminf(fminf(mny0, mny1), INFINITY),
+            win[a + (N - 1) * bb] = Box{ fminf(fminf(mnx0, mnx1), INFINITY), fminf(fminf(mny0, mny1), INFINITY),
                                    fmaxf(fmaxf(mxx0, mxx1), -INFINITY), fmaxf(fmaxf(mxy0, mxy1), -INFINITY) };
         }
 }
@@ -1679,6 +1679,144 @@ carve_classify_split_kernel(const uint64_t* __restrict__ parents,
         atomicAdd(tests_out, (unsigned long long)tsum);
 }
 
+// The smallest levels: a lane per parent, child and camera.  A level of a few hundred parents leaves most of the chip
+// idle whatever its split, and its time is the chain of one lane: the split kernel's projects 27 lattice points and
+// reads 8 windows per camera.  Here the 8 wavefronts of a block take a child each (8 points and a window per camera),
+// and the lanes of a wavefront G cameras of 64 / G parents; G is the power of two from 8 that holds the scenes'
+// cameras, 64 at most.  Points shared by children are projected again, so it only pays while the chip has room, up to
+// about kChildWaves wavefronts (split kernel of 64 lanes -> this one, us; 437 parents of 8 cameras 15.9 -> 8.5, 1891
+// 17.1 -> 9.6; 421 of 50 31 -> 21; 1523 of 64, 12184 wavefronts, 55 -> 57; 7396 of 50 93 -> 128).
+constexpr int kChildThreads = 512;
+constexpr uint64_t kChildWaves = 8192;
+
+template <bool PARTIAL, bool GL>
+__device__ __forceinline__ bool
+child_camera(const SceneDev& s, const float (&wx)[2], const float (&wy)[2], const float (&wz)[2], int32_t b, bool last,
+             uint32_t& refine, uint32_t& inside)
+{
+    const uint32_t ld = uint32_t(integral_pitch(s.W));
+    const CarveCamera cam = load_camera(s.transforms + 16 * b, GL);
+    Box lo[1], hi[1];
+    uint32_t n0 = 0u, n1 = 0u;
+    lattice_slice<GL>(cam, wx, wy, wz[0], lo, n0);
+    lattice_slice<GL>(cam, wx, wy, wz[1], hi, n1);
+    const PixelBox bb = pixel_box<GL>(box_merge(lo[0], hi[0]), float(s.W), float(s.H));
+    ChildWindow cw;
+    child_window<PARTIAL>(bb, s.integral + int64_t(b) * integral_rows(s.H) * ld, ld, float(s.H - 1), float(s.W - 1), cw);
+    const bool in = PARTIAL && last && (n0 | n1) == 0u && bb.minx >= 0.5f && bb.miny >= 0.5f &&
+                    bb.ux < float(s.W) - 1.0f && bb.uy < float(s.H) - 1.0f;
+    return child_decide<PARTIAL>(cw, in, 1u, refine, inside);
+}
+
+// One child by the lanes of its group (j of G): the group takes its cameras in rounds, as in classify_split.
+template <bool PARTIAL, bool GL>
+__device__ __forceinline__ void
+classify_child(const SceneDev& s, uint64_t key, int32_t level_i, uint32_t c, int32_t j, int32_t G, uint32_t& refine,
+               uint32_t& inside, uint32_t& first_empty)
+{
+    const float inv = __builtin_ldexpf(1.0f, -(level_i + 1));
+    float wx[2], wy[2], wz[2];
+#pragma unroll
+    for (uint32_t u = 0; u < 2; ++u)
+    {
+        wx[u] = grid_to_world(2 * key_x(key) + (c & 1u) + u, inv, s.length, s.corner[0]);
+        wy[u] = grid_to_world(2 * key_y(key) + ((c >> 1) & 1u) + u, inv, s.length, s.corner[1]);
+        wz[u] = grid_to_world(2 * key_z(key) + (c >> 2) + u, inv, s.length, s.corner[2]);
+    }
+    const bool last = level_i == s.level - 1;
+    for (int32_t b0 = 0; b0 < s.B && first_empty == 0xffffffffu; b0 += G)
+    {
+        const int32_t b = b0 + j;
+        if (b < s.B && child_camera<PARTIAL, GL>(s, wx, wy, wz, b, last, refine, inside))
+            first_empty = uint32_t(b);
+        for (int off = G / 2; off >= 1; off >>= 1)
+            first_empty = min(first_empty, uint32_t(__shfl_xor(int(first_empty), off, 64)));
+    }
+}
+
+__device__ __forceinline__ void
+child_scene(const SceneDev& s, uint64_t key, int32_t step, uint32_t c, int32_t j, int32_t G, uint32_t& occupied,
+            uint32_t& tests)
+{
+    const int32_t level_i = step - s.start;
+    if (level_i >= s.level)
+        return;
+    uint32_t refine = 0u, inside = 0u, first_empty = 0xffffffffu;
+    if (s.partial != 0)
+    {
+        if (s.opengl)
+            classify_child<true, true>(s, key, level_i, c, j, G, refine, inside, first_empty);
+        else
+            classify_child<true, false>(s, key, level_i, c, j, G, refine, inside, first_empty);
+    }
+    else
+    {
+        if (s.opengl)
+            classify_child<false, true>(s, key, level_i, c, j, G, refine, inside, first_empty);
+        else
+            classify_child<false, false>(s, key, level_i, c, j, G, refine, inside, first_empty);
+    }
+    for (int off = G / 2; off >= 1; off >>= 1)
+    {
+        refine |= uint32_t(__shfl_xor(int(refine), off, 64));
+        inside |= uint32_t(__shfl_xor(int(inside), off, 64));
+    }
+    const bool dead = first_empty != 0xffffffffu;
+    tests = dead ? first_empty + 1u : uint32_t(s.B);
+    occupied = dead ? 0u : refine;
+    if (s.partial != 0 && level_i == s.level - 1)
+        occupied &= inside;
+}
+
+__global__ __launch_bounds__(kChildThreads) void
+carve_classify_child_kernel(const uint64_t* __restrict__ parents, uint32_t n, int32_t step,
+                            const SceneDev* __restrict__ scenes, int32_t G, uint8_t* __restrict__ child_mask,
+                            unsigned long long* __restrict__ tests_out,
+                            const unsigned long long* __restrict__ dev_n) // optional: n = min(n, *dev_n)
+{
+    __shared__ uint32_t found[8][8]; // child, group: tests * 2 + occupied
+    if (dev_n != nullptr)
+        n = uint32_t(min((unsigned long long)n, *dev_n));
+    const uint32_t per = 64u / uint32_t(G), p0 = blockIdx.x * per;
+    if (p0 >= n)
+        return;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t c = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
+    const uint32_t group = lane / uint32_t(G), p = p0 + group;
+    const int32_t j = int32_t(lane & uint32_t(G - 1));
+    uint32_t occupied = 0u, tests = 0u;
+    if (p < n)
+    {
+        const uint64_t key = parents[p];
+        const uint32_t sid = key_scene(key), s0 = __builtin_amdgcn_readfirstlane(sid);
+        if (__all(sid == s0))
+            child_scene(wave_uniform(scenes[s0]), key, step, c, j, G, occupied, tests);
+        else
+            child_scene(scenes[sid], key, step, c, j, G, occupied, tests);
+    }
+    if (j == 0)
+        found[c][group] = 2u * tests + occupied;
+    __syncthreads();
+    if (threadIdx.x >= 64u)
+        return;
+    uint32_t sum = 0u;
+    if (lane < per && p0 + lane < n)
+    {
+        uint32_t mask = 0u;
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; ++k)
+        {
+            const uint32_t f = found[k][lane];
+            mask |= (f & 1u) << k;
+            sum += f >> 1;
+        }
+        child_mask[p0 + lane] = uint8_t(mask);
+    }
+    sum = __reduce_add_sync(0xffffffffffffffffull, sum);
+    if (lane == 0 && tests_out != nullptr)
+        atomicAdd(tests_out, (unsigned long long)sum);
+}
+
 __device__ __forceinline__ uint32_t
 popc4(const uint4& v)
 {
@@ -1817,7 +1955,7 @@ carve_scatter_kernel(const uint64_t* __restrict__ parents,
 // Count, scan and scatter of a level of at most kCompactParents in one launch: every block sums the masks of all
 // parents before its own (a byte each, a few 16-byte loads per thread from L2), so no block waits for another, and
 // the last one has the total for the host.  Small levels spend their time in launches: a level-7 hull of 8 cameras
-// 420 -> 384 us, a level-8 one of 16 540 -> 487.  At kCompactParents a thread reads 32 groups of masks at most.
+// 420 -> 384 us, a level-8 one of 10 540 -> 487.  At kCompactParents a thread reads 32 groups of masks at most.
 __global__ __launch_bounds__(kCarveThreads) void
 carve_compact_kernel(const uint64_t* __restrict__ parents, uint32_t n, const uint8_t* __restrict__ child_mask,
                      uint64_t* __restrict__ children, int32_t child_step, const SceneDev* __restrict__ scenes,
@@ -1852,6 +1990,16 @@ carve_compact_kernel(const uint64_t* __restrict__ parents, uint32_t n, const uin
                    mark_leaves);
 }
 
+// Lanes per parent and child of the kernel for the smallest levels, 0: too many wavefronts for it.
+static int32_t
+child_lanes(uint32_t n, int32_t max_cameras)
+{
+    int32_t G = 8;
+    while (G < max_cameras && G < 64)
+        G *= 2;
+    return uint64_t(n) * uint64_t(G) / 8u <= kChildWaves ? G : 0;
+}
+
 int32_t
 launch_carve_classify(const uint64_t* parents,
                       uint32_t n,
@@ -1861,6 +2009,7 @@ launch_carve_classify(const uint64_t* parents,
                       uint32_t* block_counts,
                       unsigned long long* tests,
                       const CarveTuning& tune,
+                      int32_t max_cameras,
                       hipStream_t st,
                       const unsigned long long* dev_n,
                       int32_t split_hint,
@@ -1869,7 +2018,14 @@ launch_carve_classify(const uint64_t* parents,
 {
     if (n == 0)
         return 0;
-    const int32_t split = dev_n != nullptr ? split_hint : carve_split_factor(n, tune);
+    int32_t split = dev_n != nullptr ? split_hint : carve_split_factor(n, tune);
+    const int32_t G = split == 64 ? child_lanes(n, max_cameras) : 0;
+    // fewer lanes when they still hold a parent's cameras in one round: the others would idle (8197 parents of 8
+    // cameras: 64 lanes 38 us, 16 15; 7421 of 10: 38, 21)
+    if (split == 64 && G == 0 && max_cameras <= 16)
+        split = 16;
+    if (split == 16 && max_cameras <= 4)
+        split = 4;
     const uint64_t nb = blocks_for(n, kCarveThreads);
     const auto count = [&] {
         if (counts)
@@ -1885,7 +2041,14 @@ launch_carve_classify(const uint64_t* parents,
         THULL_LAUNCH_CHECK();
         return split;
     }
-    if (split == 64)
+    if (G > 0)
+    {
+        carve_classify_child_kernel<<<blocks_for(n, 64 / G), kChildThreads, 0, st>>>(parents, n, level_i, scenes, G,
+                                                                                     child_mask, tests, dev_n);
+        THULL_LAUNCH_CHECK();
+        count();
+    }
+    else if (split == 64)
     {
         carve_classify_split_kernel<64><<<blocks_for(int64_t(n) * 64, 256), 256, 0, st>>>(parents, n, level_i, scenes,
                                                                                           child_mask, tests, dev_n);
