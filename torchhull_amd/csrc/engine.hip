@@ -1172,8 +1172,8 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
     if (by_bricks)
         launch_group_flags(scenes, n, most_flags, st);
     // dilation + tile popcount sums, scan of the sums, then word prefixes + vertex keys
-    const uint32_t wblocks = scan_blocks(total_words);
-    uint32_t* wsums = pool.alloc<uint32_t>(scan_sums_room(total_words));
+    const uint32_t wblocks = by_bricks ? scan_blocks(total_words) : vertex_tiles(total_words);
+    uint32_t* wsums = pool.alloc<uint32_t>(std::max((wblocks + 3u) & ~3u, 4u)); // scanned in groups of 4
     uint64_t* filled = by_bricks ? pool.alloc<uint64_t>(filled_words(total_words)) : nullptr;
     if (by_bricks)
         launch_dilate_groups(bitmap, total_words, dev_word_begin, scenes, n, wsums, filled, st);

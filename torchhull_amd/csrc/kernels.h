@@ -86,8 +86,9 @@ void launch_carve_compact(const uint64_t* parents, uint32_t n, const uint8_t* ch
 // Sets the root cell of every level-0 scene among scenes first .. first + nscenes - 1.
 void launch_mark_root_cells(const SceneDev* scenes, int32_t first, int32_t nscenes, hipStream_t st);
 // Vertex bitmap (all words, no clearing needed) = leaf cells dilated by {0,1}^3.
-// Also writes the popcount sum of every scan tile of words to block_sums
-// (scan_blocks(nwords) entries), the first pass of the vertex numbering.
+// Also writes the popcount sum of every tile of words to block_sums
+// (vertex_tiles(nwords) entries), the first pass of the vertex numbering.
+uint32_t vertex_tiles(uint64_t nwords);
 void launch_dilate_cells(uint32_t* verts, uint64_t nwords, const uint64_t* scene_word_begin, const SceneDev* scenes,
                          int32_t nscenes, uint32_t* block_sums, hipStream_t st);
 

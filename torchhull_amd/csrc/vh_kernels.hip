@@ -2233,10 +2233,17 @@ dilate_combine(const DilateReads& d, bool lane0)
     return out;
 }
 
-// Each block covers kScanTile consecutive words, each thread one word per
-// 256, in batches of 4 words whose reads are in flight together.  The block
+// Each block covers a tile of 256 ITEMS consecutive words, each thread one word per
+// 256, in batches of up to 4 words whose reads are in flight together.  The block
 // also sums the popcounts of its words: the first pass of the exclusive scan
-// that numbers the vertices (the tile is that of the scan's down-sweep).
+// that numbers the vertices.  Small bitmaps take 2 words per thread, so that there
+// are blocks for the chip (dilation + numbering, us, with 16 -> 2: level 7, 84 000
+// words, 16 + 20 -> 5 + 6; level 9, 4.5 million, 26 + 32 -> 24 + 22; level 10, 36
+// million, 122 + 139 -> 161 + 158).
+constexpr int kVertexItems = 2;
+constexpr uint64_t kSmallTileWords = uint64_t(1) << 23;
+
+template <int ITEMS>
 __global__ __launch_bounds__(kScanThreads) void
 dilate_cells_kernel(uint32_t* __restrict__ verts,
                     uint64_t nwords,
@@ -2245,9 +2252,9 @@ dilate_cells_kernel(uint32_t* __restrict__ verts,
                     int32_t nscenes,
                     uint32_t* __restrict__ block_sums)
 {
-    constexpr int kBatch = 4;
+    constexpr int kBatch = ITEMS < 4 ? ITEMS : 4;
     __shared__ uint32_t lds[kScanThreads / 64];
-    const uint64_t w0 = uint64_t(blockIdx.x) * kScanTile + threadIdx.x;
+    const uint64_t w0 = uint64_t(blockIdx.x) * (kScanThreads * ITEMS) + threadIdx.x;
     const bool lane0 = (threadIdx.x & 63) == 0;
     const auto begin = [&](int32_t i) { return scene_word_begin[i]; };
     // all lanes take part in the lookup ballot before any diverge
@@ -2259,7 +2266,7 @@ dilate_cells_kernel(uint32_t* __restrict__ verts,
     WordPos q{ 0u, 0u, 0u };   // position of the previous word of this thread in scene `at`
     uint32_t step_w = 0u, step_r = 0u, R1 = 0u, rw = 0u;
     uint32_t count = 0u;
-    for (int k0 = 0; k0 < kScanItems; k0 += kBatch)
+    for (int k0 = 0; k0 < ITEMS; k0 += kBatch)
     {
         DilateReads d[kBatch];
 #pragma unroll
@@ -2345,19 +2352,27 @@ launch_dilate_cells(uint32_t* verts, uint64_t nwords, const uint64_t* scene_word
 {
     if (nwords == 0)
         return;
-    dilate_cells_kernel<<<scan_blocks(nwords), kScanThreads, 0, st>>>(verts, nwords, scene_word_begin, scenes, nscenes,
-                                                                      block_sums);
+    const auto kernel = nwords <= kSmallTileWords ? dilate_cells_kernel<kVertexItems> : dilate_cells_kernel<kScanItems>;
+    kernel<<<vertex_tiles(nwords), kScanThreads, 0, st>>>(verts, nwords, scene_word_begin, scenes, nscenes, block_sums);
     THULL_LAUNCH_CHECK();
 }
 
+uint32_t
+vertex_tiles(uint64_t nwords)
+{
+    const uint64_t tile = nwords <= kSmallTileWords ? kScanThreads * kVertexItems : kScanTile;
+    return uint32_t((nwords + tile - 1) / tile);
+}
+
 // Second pass of the vertex numbering fused with the vertex extraction.  Wave
-// w of a block takes the block's words [w * 1024, (w + 1) * 1024) in 16 steps
-// of 64 consecutive words (one per lane, coalesced); a wave prefix sum of
+// w of a block takes the block's words [w * 64 ITEMS, (w + 1) * 64 ITEMS) in ITEMS
+// steps of 64 consecutive words (one per lane, coalesced); a wave prefix sum of
 // the popcounts plus a running total turn the block offsets of the dilation
 // pass into the exclusive prefix of every word (stored for the marching-cubes
 // rank lookups), and each set bit's packed key is written at prefix[word] +
 // rank, i.e. in bitmap order = per scene (z, y, x) order; adjacent lanes write
 // adjacent keys.
+template <int ITEMS>
 __global__ __launch_bounds__(kScanThreads) void
 prefix_extract_kernel(const uint32_t* __restrict__ bitmap,
                       uint64_t nwords,
@@ -2368,11 +2383,10 @@ prefix_extract_kernel(const uint32_t* __restrict__ bitmap,
                       uint32_t* __restrict__ prefix,
                       uint64_t* __restrict__ vertices)
 {
-    constexpr int kWaveWords = kScanTile / (kScanThreads / 64);
-    constexpr int kSteps = kWaveWords / 64;
+    constexpr int kSteps = ITEMS, kWaveWords = 64 * ITEMS;
     __shared__ uint32_t wave_total[kScanThreads / 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint64_t wbase = uint64_t(blockIdx.x) * kScanTile + uint64_t(wave) * kWaveWords;
+    const uint64_t wbase = uint64_t(blockIdx.x) * (kScanThreads * ITEMS) + uint64_t(wave) * kWaveWords;
     uint32_t v[kSteps];
     uint32_t total = 0;
 #pragma unroll
@@ -2453,9 +2467,10 @@ launch_prefix_extract(const uint32_t* bitmap,
 {
     if (nwords == 0)
         return;
-    prefix_extract_kernel<<<scan_blocks(nwords), kScanThreads, 0, st>>>(bitmap, nwords, block_offsets,
-                                                                        scene_word_begin, scenes, nscenes, prefix,
-                                                                        vertices);
+    const auto kernel =
+            nwords <= kSmallTileWords ? prefix_extract_kernel<kVertexItems> : prefix_extract_kernel<kScanItems>;
+    kernel<<<vertex_tiles(nwords), kScanThreads, 0, st>>>(bitmap, nwords, block_offsets, scene_word_begin, scenes,
+                                                          nscenes, prefix, vertices);
     THULL_LAUNCH_CHECK();
 }
 
