@@ -237,7 +237,7 @@ class HostNotify
 public:
     HostNotify()
     {
-        THULL_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_), 4 * sizeof(unsigned long long),
+        THULL_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_), (4 + kTable) * sizeof(unsigned long long),
                                 hipHostMallocCoherent | hipHostMallocMapped));
         const hipError_t e = hipHostGetDevicePointer(reinterpret_cast<void**>(&dev_), host_, 0);
         if (e != hipSuccess)
@@ -257,6 +257,11 @@ public:
     {
         return ScanNotify{ dev_, extra, ++seq_ };
     }
+
+    // Words that a kernel may write ahead of its notification.
+    static constexpr int kTable = 3 * 256;
+    unsigned long long* dev_table() const { return dev_ + 4; }
+    const unsigned long long* table() const { return host_ + 4; }
 
     // Waits for the notification `n` (queued on `st`); false when the stream went idle without it,
     // and the caller then reads the values from device memory.
@@ -561,8 +566,9 @@ struct LoadPopcountMask
     __device__ uint32_t operator()(uint64_t i) const { return __popc(m[i] & 7u); }
 };
 
-// Per scene: first vertex position, first output vertex and first triangle-vertex.
-__global__ void
+// Per scene: first vertex position, first output vertex and first triangle-vertex, the latter two also as the tables of
+// the faces kernel.  One block sends them, after the two totals, to the host by `note` and `host_out`.
+__global__ __launch_bounds__(256) void
 scene_starts_kernel(const uint64_t* word_begin,
                     int32_t n,
                     uint64_t nwords,
@@ -572,24 +578,47 @@ scene_starts_kernel(const uint64_t* word_begin,
                     const uint32_t* tbase,
                     const unsigned long long* totals, // triangle vertices, output vertices (unique meshes)
                     bool unique,
-                    unsigned long long* out)
+                    unsigned long long* out,
+                    uint32_t* vstart,
+                    uint32_t* tstart,
+                    unsigned long long* host_out, // with note: one block, n < 256
+                    ScanNotify note)
 {
     const int32_t s = blockIdx.x * 256 + threadIdx.x;
-    if (s > n)
-        return;
     const uint64_t ttotal = totals[0], vtotal = unique ? totals[1] : ttotal;
-    uint64_t first = nverts;
-    if (s < n && word_begin[s] < nwords)
-        first = bitmap_prefix[word_begin[s]];
-    uint64_t vs = vtotal, ts = ttotal;
-    if (first < nverts)
+    if (s <= n)
     {
-        ts = tbase[first];
-        vs = vbase != nullptr ? vbase[first] : ts; // soup vertices sit at the triangle-vertex slots
+        uint64_t first = nverts;
+        if (s < n && word_begin[s] < nwords)
+            first = bitmap_prefix[word_begin[s]];
+        uint64_t vs = vtotal, ts = ttotal;
+        if (first < nverts)
+        {
+            ts = tbase[first];
+            vs = vbase != nullptr ? vbase[first] : ts; // soup vertices sit at the triangle-vertex slots
+        }
+        out[3 * s + 0] = first;
+        out[3 * s + 1] = vs;
+        out[3 * s + 2] = ts;
+        if (note.slot != nullptr)
+        {
+            host_out[3 * s + 0] = first;
+            host_out[3 * s + 1] = vs;
+            host_out[3 * s + 2] = ts;
+        }
+        vstart[s] = uint32_t(vs);
+        tstart[s] = uint32_t(ts);
     }
-    out[3 * s + 0] = first;
-    out[3 * s + 1] = vs;
-    out[3 * s + 2] = ts;
+    if (note.slot == nullptr)
+        return;
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0)
+    {
+        note.slot[0] = ttotal;
+        note.slot[1] = vtotal;
+        __hip_atomic_store(note.slot + 2, note.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 __global__ void
@@ -815,7 +844,19 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
     int32_t last_step = 0; // carving steps the run needs: max over scenes of start + level
     uint32_t* first_cells = nullptr; // leaf-cell bitmaps of the initial scenes
     uint64_t first_cell_words = 0;
-    SceneDev* scenes = pool.alloc<SceneDev>(capacity);
+    // descriptors, roots, first words and grids: one block, which goes up in one copy when no scene can join (a small
+    // hull spends most of its time between launches; with the starts sent by their kernel, 9 copies, 2 launches and a
+    // stream synchronisation less: a level-7 hull of 8 cameras 351 -> 294 us)
+    static_assert(sizeof(SceneDev) % 8 == 0 && alignof(SceneDev) <= 8 && alignof(McGrid) <= 8, "table of 8-byte parts");
+    const size_t room_all = size_t(std::max(capacity, 1));
+    SceneDev* scenes = reinterpret_cast<SceneDev*>(pool.alloc_bytes(
+            room_all * (sizeof(SceneDev) + 2 * sizeof(uint64_t) + sizeof(McGrid)) + sizeof(uint64_t)));
+    uint64_t* const root_list = reinterpret_cast<uint64_t*>(scenes + room_all);
+    uint64_t* const dev_word_begin = root_list + room_all;
+    McGrid* const dgrids = reinterpret_cast<McGrid*>(dev_word_begin + room_all + 1);
+    // camera-test counters of every carving step (a joined scene ends by the last step), cleared with the first cells
+    constexpr int32_t kMaxSteps = 64;
+    unsigned long long* dev_tests = nullptr;
     unsigned long long* dev_total = pool.alloc<unsigned long long>(2);
 
     // Adds scenes k0 .. all.size() - 1, which start at carving step `start`: descriptors, integral images
@@ -826,6 +867,27 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
     // cells.  Each scene's own cells keep the reference's parent-major order, so no result depends on it.
     const bool by_bricks = solid_maps_pay(in, n0);
     uint64_t most_flags = 0;
+    // marching-cubes grids of all scenes: isolevel 0.5, world coordinates, flipped faces
+    const auto scene_grids = [&] {
+        std::vector<McGrid> grids(all.size());
+        for (size_t s = 0; s < all.size(); ++s)
+        {
+            McGrid g{};
+            const uint32_t R1 = (1u << std::max(0, all[s].level)) + 1u;
+            g.dims[0] = g.dims[1] = g.dims[2] = R1;
+            g.row_words = sd[s].row_words;
+            g.bitmap_offset = sd[s].bitmap_offset;
+            g.out_mode = 2;
+            const float scale = all[s].cube_length / float(int64_t(1) << std::max(0, all[s].level));
+            g.scale[0] = g.scale[1] = g.scale[2] = scale;
+            g.corner[0] = all[s].cube_corner_bfl[0];
+            g.corner[1] = all[s].cube_corner_bfl[1];
+            g.corner[2] = all[s].cube_corner_bfl[2];
+            g.flip = 1;
+            grids[s] = g;
+        }
+        return grids;
+    };
     auto add_scenes = [&](size_t k0, int32_t start) {
         const size_t k1 = all.size();
         std::vector<IntegralRequest> ireq;
@@ -898,8 +960,12 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
             sd[s].group_flags = pool.alloc<uint8_t>(flags);
             most_flags = std::max(most_flags, flags);
         }
-        uint32_t* cells = pool.alloc<uint32_t>(std::max<uint64_t>(cell_words + brick_words, 1));
-        launch_fill_u32(cells, cell_words + brick_words, 0u, st);
+        const uint64_t test_words = k0 == 0 ? 2 * kMaxSteps : 0; // keep the cells' alignment
+        uint32_t* cells = pool.alloc<uint32_t>(std::max<uint64_t>(test_words + cell_words + brick_words, 1));
+        launch_fill_u32(cells, test_words + cell_words + brick_words, 0u, st);
+        if (k0 == 0)
+            dev_tests = reinterpret_cast<unsigned long long*>(cells);
+        cells += test_words;
         for (size_t s = k0, w = cell_words; by_bricks && s < k1; ++s)
         {
             sd[s].bricks = cells + w;
@@ -923,8 +989,6 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
                                       pool.alloc<float>(std::max<uint64_t>(carry_floats, 1)),
                                       pool.alloc_bytes(integral_job_bytes(std::max<size_t>(ireq.size(), 1))),
                                       pool.alloc_bytes(solid_job_bytes(ireq.size())), ctx.upload, st);
-        ctx.upload.upload(scenes + k0, sd.data() + k0, (k1 - k0) * sizeof(SceneDev), st);
-        launch_mark_root_cells(scenes, int32_t(k0), int32_t(k1 - k0), st);
         std::vector<int32_t> order;
         for (size_t s = k0; s < k1; ++s)
             order.push_back(int32_t(s));
@@ -934,22 +998,35 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
         std::vector<uint64_t> roots(order.size());
         for (size_t k = 0; k < order.size(); ++k)
             roots[k] = pack_key(uint32_t(order[k]), 0, 0, 0);
+        if (join == nullptr)
+        {
+            word_begin.push_back(total_words);
+            const std::vector<McGrid> grids = scene_grids();
+            std::vector<char> table;
+            const auto put = [&](const void* p, size_t bytes) {
+                table.insert(table.end(), static_cast<const char*>(p), static_cast<const char*>(p) + bytes);
+            };
+            put(sd.data(), sd.size() * sizeof(SceneDev));
+            put(roots.data(), roots.size() * sizeof(uint64_t));
+            put(word_begin.data(), word_begin.size() * sizeof(uint64_t));
+            put(grids.data(), grids.size() * sizeof(McGrid));
+            ctx.upload.upload(scenes, table.data(), table.size(), st);
+        }
+        else
+            ctx.upload.upload(scenes + k0, sd.data() + k0, (k1 - k0) * sizeof(SceneDev), st);
+        if (std::any_of(sd.begin() + k0, sd.end(), [](const SceneDev& d) { return d.level == 0; }))
+            launch_mark_root_cells(scenes, int32_t(k0), int32_t(k1 - k0), st);
         return roots;
     };
 
     all.assign(in, in + n0);
     std::vector<uint64_t> roots = add_scenes(0, 0);
-    // room for the roots of scenes that may still join
-    uint64_t* list = pool.alloc<uint64_t>(std::max<size_t>(size_t(capacity), 1));
-    ctx.upload.upload(list, roots.data(), roots.size() * sizeof(uint64_t), st);
+    uint64_t* list = root_list; // with room for the roots of scenes that may still join
+    if (join != nullptr)
+        ctx.upload.upload(list, roots.data(), roots.size() * sizeof(uint64_t), st);
     uint32_t count = uint32_t(roots.size());
     ctx.level_lists.push_back(list);
     ctx.level_sizes.push_back(count);
-
-    // camera-test counters of every carving step, cleared once (a joined scene ends by the last step)
-    constexpr int32_t kMaxSteps = 64;
-    unsigned long long* dev_tests = pool.alloc<unsigned long long>(kMaxSteps);
-    launch_fill_u32(reinterpret_cast<uint32_t*>(dev_tests), 2 * kMaxSteps, 0u, st);
 
     // ---- replay of the captured carving loop of this batch shape (thull_ctx_set_graph_replay) ----
     const bool graph = ctx.graph_replay && join == nullptr;
@@ -1140,13 +1217,17 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
     if (graph && !replayed)
         make_plan(ctx, sig, roots, last_step, st);
     const int32_t n = int32_t(all.size());
-    word_begin.push_back(total_words);
     ctx.scenes_host = sd;
     const int32_t nlists = int32_t(ctx.level_lists.size());
 
     // ---- corner vertices (VH:770-825): leaf cells (marked above), then their corners by dilation ----
-    uint64_t* dev_word_begin = pool.alloc<uint64_t>(n + 1);
-    ctx.upload.upload(dev_word_begin, word_begin.data(), (n + 1) * sizeof(uint64_t), st);
+    if (join != nullptr)
+    {
+        word_begin.push_back(total_words);
+        const std::vector<McGrid> grids = scene_grids();
+        ctx.upload.upload(dev_word_begin, word_begin.data(), (n + 1) * sizeof(uint64_t), st);
+        ctx.upload.upload(dgrids, grids.data(), n * sizeof(McGrid), st);
+    }
     uint32_t* bitmap = pool.alloc<uint32_t>(std::max<uint64_t>(total_words, 1));
     uint32_t* prefix = pool.alloc<uint32_t>(std::max<uint64_t>(total_words, 1));
     std::vector<BrickList> bricks; // lists of the steps at which some scene's bricks are kept
@@ -1205,26 +1286,7 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
     ctx.vertices = vertices;
     ctx.values = values;
 
-    // ---- sparse marching cubes at isolevel 0.5, world coordinates, flipped faces ----
-    std::vector<McGrid> grids(n);
-    for (int32_t s = 0; s < n; ++s)
-    {
-        McGrid g{};
-        const uint32_t R1 = (1u << std::max(0, all[s].level)) + 1u;
-        g.dims[0] = g.dims[1] = g.dims[2] = R1;
-        g.row_words = sd[s].row_words;
-        g.bitmap_offset = sd[s].bitmap_offset;
-        g.out_mode = 2;
-        const float scale = all[s].cube_length / float(int64_t(1) << std::max(0, all[s].level));
-        g.scale[0] = g.scale[1] = g.scale[2] = scale;
-        g.corner[0] = all[s].cube_corner_bfl[0];
-        g.corner[1] = all[s].cube_corner_bfl[1];
-        g.corner[2] = all[s].cube_corner_bfl[2];
-        g.flip = 1;
-        grids[s] = g;
-    }
-    McGrid* dgrids = pool.alloc<McGrid>(n);
-    ctx.upload.upload(dgrids, grids.data(), n * sizeof(McGrid), st);
+    // ---- sparse marching cubes ----
     McPlan plan{};
     plan.grids = dgrids;
     plan.vertices = vertices;
@@ -1257,36 +1319,35 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
             exclusive_scan(LoadPopcountMask{ emask }, nverts, vbase, sums, dev_total + 1, st);
         }
         unsigned long long* dstarts = pool.alloc<unsigned long long>(3 * (n + 1));
-        scene_starts_kernel<<<blocks_for(n + 1, 256), 256, 0, st>>>(dev_word_begin, n, total_words, prefix, nverts,
-                                                                    vbase, tbase, dev_total, unique, dstarts);
-        THULL_LAUNCH_CHECK();
+        uint32_t* dv = pool.alloc<uint32_t>(n + 1);
+        uint32_t* dt = pool.alloc<uint32_t>(n + 1);
         // one wait for the two totals and the scene starts
-        const size_t words = 2 + starts.size();
-        std::vector<unsigned long long> big;
-        unsigned long long* h = ctx.stage->p;
-        if (words > size_t(HostStage::kSlots))
+        const bool notes = 3 * (n + 1) <= HostNotify::kTable;
+        const ScanNotify note = notes ? ctx.notify.next(nullptr) : ScanNotify{};
+        scene_starts_kernel<<<blocks_for(n + 1, 256), 256, 0, st>>>(dev_word_begin, n, total_words, prefix, nverts,
+                                                                    vbase, tbase, dev_total, unique, dstarts, dv, dt,
+                                                                    ctx.notify.dev_table(), note);
+        THULL_LAUNCH_CHECK();
+        unsigned long long got[2];
+        if (notes && ctx.notify.wait(note, st, got))
         {
-            big.resize(words);
-            h = big.data();
+            std::copy(ctx.notify.table(), ctx.notify.table() + starts.size(), starts.begin());
+            ttotal = got[0];
         }
-        THULL_HIP(hipMemcpyAsync(h, dev_total, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
-        THULL_HIP(hipMemcpyAsync(h + 2, dstarts, starts.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                                 st));
-        THULL_HIP(hipStreamSynchronize(st));
-        ttotal = h[0];
-        vtotal = unique ? h[1] : ttotal;
+        else
+        {
+            THULL_HIP(hipMemcpyAsync(starts.data(), dstarts, starts.size() * sizeof(unsigned long long),
+                                     hipMemcpyDeviceToHost, st));
+            ttotal = ctx.read_u64(dev_total, st);
+        }
+        vtotal = unique ? starts[3 * n + 1] : ttotal; // the entries past the last scene are the totals
         check_u32(ttotal, "triangle vertex count");
-        std::copy(h + 2, h + words, starts.begin());
         std::vector<uint32_t> vstart(n + 1), tstart(n + 1);
         for (int32_t s = 0; s <= n; ++s)
         {
             vstart[s] = uint32_t(starts[3 * s + 1]);
             tstart[s] = uint32_t(starts[3 * s + 2]);
         }
-        uint32_t* dv = pool.alloc<uint32_t>(n + 1);
-        uint32_t* dt = pool.alloc<uint32_t>(n + 1);
-        ctx.upload.upload(dv, vstart.data(), (n + 1) * sizeof(uint32_t), st);
-        ctx.upload.upload(dt, tstart.data(), (n + 1) * sizeof(uint32_t), st);
         verts = pool.alloc<float>(3 * std::max<uint64_t>(vtotal, 1));
         faces = pool.alloc<int64_t>(std::max<uint64_t>(ttotal, 1));
         if (unique)
