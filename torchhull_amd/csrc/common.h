@@ -324,7 +324,7 @@ struct SceneDev
     uint32_t* bricks;
     uint8_t* group_flags; // with bricks: flags of the groups of 4 words of the vertex bitmap (group_flags_kernel)
     int32_t brick_shift;
-    int32_t pad_;
+    int32_t culls; // set by the solid map pass: some camera's CullCamera::reach lets carving skip it
 };
 
 // Bricks of the field are at most 8 cells per side.

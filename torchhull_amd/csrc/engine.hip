@@ -937,6 +937,7 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
                     r.solid = pool.alloc<uint8_t>(solid_map_bytes(sc.B, sc.H, sc.W));
                     r.cull = pool.alloc<CullCamera>(uint64_t(sc.B));
                     r.solid_scratch = pool.alloc_bytes(solid_scratch_bytes(sc.B, sc.H, sc.W));
+                    r.culls = &scenes[s].culls;
                     r.transforms = sc.transforms;
                     r.opengl = sc.opengl;
                     std::copy(sc.cube_corner_bfl, sc.cube_corner_bfl + 3, r.corner);
@@ -982,13 +983,6 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
             sd[s].cells = cells + off;
             off += ((uint64_t(1) << (2 * sd[s].level)) * sd[s].cell_row_words + 3) & ~uint64_t(3);
         }
-        uint64_t carry_floats = 0;
-        for (const auto& r : ireq)
-            carry_floats += integral_carry_floats(r.B, r.H, r.W);
-        launch_integral_images_padded(ireq.data(), int32_t(ireq.size()),
-                                      pool.alloc<float>(std::max<uint64_t>(carry_floats, 1)),
-                                      pool.alloc_bytes(integral_job_bytes(std::max<size_t>(ireq.size(), 1))),
-                                      pool.alloc_bytes(solid_job_bytes(ireq.size())), ctx.upload, st);
         std::vector<int32_t> order;
         for (size_t s = k0; s < k1; ++s)
             order.push_back(int32_t(s));
@@ -1014,6 +1008,14 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
         }
         else
             ctx.upload.upload(scenes + k0, sd.data() + k0, (k1 - k0) * sizeof(SceneDev), st);
+        // after the descriptors: the solid map pass sets SceneDev::culls
+        uint64_t carry_floats = 0;
+        for (const auto& r : ireq)
+            carry_floats += integral_carry_floats(r.B, r.H, r.W);
+        launch_integral_images_padded(ireq.data(), int32_t(ireq.size()),
+                                      pool.alloc<float>(std::max<uint64_t>(carry_floats, 1)),
+                                      pool.alloc_bytes(integral_job_bytes(std::max<size_t>(ireq.size(), 1))),
+                                      pool.alloc_bytes(solid_job_bytes(ireq.size())), ctx.upload, st);
         if (std::any_of(sd.begin() + k0, sd.end(), [](const SceneDev& d) { return d.level == 0; }))
             launch_mark_root_cells(scenes, int32_t(k0), int32_t(k1 - k0), st);
         return roots;

@@ -30,6 +30,7 @@ struct IntegralRequest
     uint8_t* solid;
     CullCamera* cull;
     void* solid_scratch;
+    int32_t* culls; // the scene's SceneDev::culls on the device
     const float* transforms;
     int32_t opengl;
     float corner[3];
