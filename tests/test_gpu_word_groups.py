@@ -50,3 +50,28 @@ def test_tiles_of_several_scenes_equal_single_calls():
     for s, (v, f) in zip(scenes, th.visual_hull_batch(scenes)):
         va, fa = th.visual_hull(**s)
         assert torch.equal(fa, f) and torch.equal(va.view(torch.int32), v.view(torch.int32))
+
+
+def test_scenes_that_join_a_loop_by_bricks_equal_single_calls():
+    # scenes handed over at level boundaries of a loop that keeps bricks: their descriptors, maps, bitmaps and flags
+    # are added while the loop runs
+    import torchhull_amd as th
+    from torchhull_amd import api
+
+    scenes = []
+    for i, (cameras, level) in enumerate(((40, 9), (12, 6), (36, 7), (5, 0), (6, 4))):
+        masks, T = _border_scene(cameras, 200, 1.0 if i % 2 else -1.0)
+        scenes.append(dict(masks=torch.from_numpy(masks).to(DEV), transforms=torch.from_numpy(T).to(DEV), level=level,
+                           cube_corner_bfl=(-1.0, -1.0, -1.0), cube_length=2.0, masks_partial=False,
+                           transforms_convention="opengl"))
+    keep: list = []
+    structs = [api._scene_struct(**s, keep=keep) for s in scenes]
+    steps = {2: [structs[1], structs[2]], 5: [structs[3], structs[4]]}
+    print("case joining scenes", flush=True)
+    run = api._Run(structs[:1], torch.device(DEV), True, join=lambda step, last, room: steps.pop(step, []),
+                   max_scenes=len(structs))
+    meshes = run.meshes()
+    assert len(meshes) == len(scenes)
+    for s, (v, f) in zip(scenes, meshes):
+        va, fa = th.visual_hull(**s)
+        assert torch.equal(fa, f) and torch.equal(va.view(torch.int32), v.view(torch.int32))
