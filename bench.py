@@ -113,7 +113,8 @@ def carve_profile(run_fn, reps: int = 5) -> dict:
     return dict(levels=levels, reps=len(runs))
 
 
-CARVE_SOURCES = ("torchhull_amd/csrc/vh_kernels.hip", "torchhull_amd/csrc/common.h", "torchhull_amd/csrc/engine.hip")
+CARVE_SOURCES = ("torchhull_amd/csrc/vh_kernels.hip", "torchhull_amd/csrc/common.h", "torchhull_amd/csrc/solid_reach.h",
+                 "torchhull_amd/csrc/engine.hip")
 
 
 def carve_source_hash() -> str:

@@ -15,6 +15,7 @@
 
 #include "kernels.h"
 #include "scan.h"
+#include "solid_reach.h"
 
 namespace thull
 {
@@ -431,25 +432,6 @@ struct SolidJob
     uint64_t begin;        // first workgroup of this job
 };
 
-// How far (in pixels from a cell's centre) a window of solid pixels may reach so that its box sum is certain to
-// classify as full.  Integral images of whole numbers below 2^23 are exact.  Otherwise the window of w columns
-// lies between two row chains that each round w times by at most half an ulp of the image's total (2^(S - 25)
-// for a total below 2^S), the column chains under it by H 2^-21 per column (an addition of 1 rounds only where it
-// crosses a power of two), and the three operations of the box sum by 2 * 2^(S - 24) in all: the sum is within
-// (w + 2) 2^(S - 24) + w H 2^-21 of the area, which has to stay clear of the margin of 0.4 (0.35 here).
-__device__ __forceinline__ float
-solid_reach(bool negative, bool fraction, float total, int32_t H)
-{
-    if (negative || !(total < 0x1p40f))
-        return -1.0f;
-    if (!fraction && total < 0x1p23f)
-        return 1e9f;
-    int e = 0;
-    (void)frexpf(total, &e); // total < 2^e
-    const float a = __builtin_ldexpf(1.0f, e - 24), c = float(H) * 0x1p-21f;
-    return (0.35f - 4.0f * a - 2.0f * c) / (2.0f * a + 2.0f * c); // w = 2 reach + 2
-}
-
 // A window reaches at least 1.75 pixels (skip_probe): below this carving can skip no camera, and the tests are left
 // out (blurred 2048^2 masks have no reach; a level-10 hull of 32 partial ones 3.75 -> 3.68 ms).
 constexpr float kLeastReach = 2.0f;
@@ -490,7 +472,7 @@ solid_map_kernel(const SolidJob* __restrict__ jobs, int32_t njobs)
         };
         CullCamera c{};
         const bool f32 = j.u8 == 0;
-        c.reach = solid_reach(f32 && __shfl(odd, 0, 64) != 0, f32 && __shfl(odd, 1, 64) != 0, total, j.H);
+        c.reach = solid_reach(f32 && __shfl(odd, 0, 64) != 0, f32 && __shfl(odd, 1, 64) != 0, total, j.H, j.W);
         c.sum_d = at(d0) + at(d0 + 1) + at(d0 + 2);
         c.ex = bound(0);
         c.ey = bound(4);
