@@ -3304,35 +3304,39 @@ field_product(const SceneDev& s, float wx, float wy, float wz, Cameras cams)
     const float pad = PARTIAL ? 1.0f : 0.0f; // ones padding (partial) or zeros padding (full), IU:162-214
     constexpr int U = 4; // cameras whose reads are in flight together
     float value = 1.0f;
-    while (cams.left() >= U)
-    {
-        if constexpr (PAIR)
-            if (cams.template inside<U>())
-            {
-                InsideSample<T> f[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u)
-                    inside_sample<T, OFF32>(s, cams.next(), wx, wy, wz, f[u]);
-#pragma unroll
-                for (int u = 0; u < U; ++u)
-                    value *= inside_factor<T>(f[u]);
-                continue;
-            }
-        FieldSample<T> f[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            field_sample<T, PAIR, PARTIAL, OFF32>(s, cams.next(), wx, wy, wz, f[u]);
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (!PARTIAL || !f[u].skip)
-                value *= field_factor<T>(f[u], pad);
-    }
     while (cams.left() > 0)
     {
-        FieldSample<T> f;
-        field_sample<T, PAIR, PARTIAL, OFF32>(s, cams.next(), wx, wy, wz, f);
-        if (!PARTIAL || !f.skip)
-            value *= field_factor<T>(f, pad);
+        while (cams.left() >= U)
+        {
+            if constexpr (PAIR)
+                if (cams.template inside<U>())
+                {
+                    InsideSample<T> f[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                        inside_sample<T, OFF32>(s, cams.next(), wx, wy, wz, f[u]);
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                        value *= inside_factor<T>(f[u]);
+                    continue;
+                }
+            FieldSample<T> f[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                field_sample<T, PAIR, PARTIAL, OFF32>(s, cams.next(), wx, wy, wz, f[u]);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (!PARTIAL || !f[u].skip)
+                    value *= field_factor<T>(f[u], pad);
+        }
+        // the rest of a camera word: the next word's cameras go U at a time again
+        for (int32_t rest = cams.left(); rest > 0; --rest)
+        {
+            FieldSample<T> f;
+            field_sample<T, PAIR, PARTIAL, OFF32>(s, cams.next(), wx, wy, wz, f);
+            if (!PARTIAL || !f.skip)
+                value *= field_factor<T>(f, pad);
+        }
     }
     return value;
 }
