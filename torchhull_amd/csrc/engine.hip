@@ -770,7 +770,8 @@ record_plan(Context& ctx, const CarvePlan& p, const std::vector<SceneDev>& sd, i
         if (timed)
             THULL_HIP(hipEventRecord(ctx.event(2 * i), st));
         launch_carve_classify(p.lists[i], p.cap[i], i, p.scenes, p.masks[i], p.bcount[i], tests + i, ctx.tuning,
-                              max_cameras(sd), st, counts + i, p.split[i], p.cursors + 8 * i);
+                              max_cameras(sd), carve_culls(sd.data(), sd.size(), i), st, counts + i, p.split[i],
+                              p.cursors + 8 * i);
         if (timed)
             THULL_HIP(hipEventRecord(ctx.event(2 * i + 1), st));
         // the next level's size, clamped to its list's capacity (overflow: the run is repeated)
@@ -1170,7 +1171,8 @@ visual_hull_run(Context& ctx, const thull_scene* in, int32_t n0, bool unique, hi
         if (ctx.profile)
             THULL_HIP(hipEventRecord(ctx.event(2 * i), st));
         const int32_t split = launch_carve_classify(list, count, i, scenes, mask, bcount, dev_tests + i, ctx.tuning,
-                                                    max_cameras(sd), st, nullptr, 0, nullptr, !compact);
+                                                    max_cameras(sd), carve_culls(sd.data(), sd.size(), i), st, nullptr,
+                                                    0, nullptr, !compact);
         if (ctx.profile)
             THULL_HIP(hipEventRecord(ctx.event(2 * i + 1), st));
         // the scan sends the next level's size (and the camera tests) to the host; the children go out

@@ -58,13 +58,16 @@ struct CarveTuning
     uint32_t max_parents[4] = { 16384u, 131072u, 1048576u, 1048576u }; // G = 64, 16, 4, 2 up to these sizes
 };
 int32_t carve_split_factor(uint32_t n, const CarveTuning& tune);
+// Whether carving of some scene may leave out cameras at a step (host descriptors).
+bool carve_culls(const SceneDev* scenes, size_t n, int32_t step);
 // `step`: the carving step (a scene's octree level is step - its start).  `max_cameras`: the most cameras of a scene.
+// `culls`: carve_culls of the launch's scenes.
 // Device-driven levels (dev_n non-null): the level holds min(*dev_n, n) parents, n being the list's
 // capacity; the lanes per parent are `split_hint`, and with one lane per parent a persistent queue
 // kernel runs (carve_classify_queue_kernel, `cursors`: 8 words, zero at start).
 int32_t launch_carve_classify(const uint64_t* parents, uint32_t n, int32_t step, const SceneDev* scenes,
                               uint8_t* child_mask, uint32_t* block_counts, unsigned long long* tests,
-                              const CarveTuning& tune, int32_t max_cameras, hipStream_t st,
+                              const CarveTuning& tune, int32_t max_cameras, bool culls, hipStream_t st,
                               const unsigned long long* dev_n = nullptr, int32_t split_hint = 0,
                               uint32_t* cursors = nullptr, bool counts = true);
 

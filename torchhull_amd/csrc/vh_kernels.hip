@@ -1279,16 +1279,23 @@ carve_skips(const SceneDev& s, int32_t b0, int32_t step, int32_t end, float half
     return skips;
 }
 
-// Whether testing the cameras of a level-li cell is worth it: cells of more than kCullPixels pixels of an image that
-// the cube about fills reach past the solid parts of the silhouettes too often.  (Share of the cameras that a
-// wavefront of 64 parents of a 50-camera 1080p hull still tests, by level of the parents: 5 97 %, 6 78 %, 7 53 %,
-// 8 38 %; levels 10 and 11 of it carve in 1.54 instead of 4.45 ms.)
+// Whether testing the cameras of a level-li cell is worth it.  A cell that is large beside the object lies on the
+// outlines of most silhouettes, so the level decides (share of the cameras that a wavefront of 64 parents of a
+// 50-camera 1080p hull still tests, by level of the parents: 5 97 %, 6 78 %, 7 53 %, 8 38 %); and a cell of more
+// pixels than the maps' distances reach past is in no map's solid part, whatever its level.
+constexpr int32_t kCullLevel = 7;
 constexpr int32_t kCullPixels = 16;
+
+__host__ __device__ __forceinline__ bool
+cull_level(const SceneDev& s, int32_t li)
+{
+    return s.solid != nullptr && li >= kCullLevel && ((s.H > s.W ? s.H : s.W) >> li) <= kCullPixels;
+}
 
 __device__ __forceinline__ bool
 cull_pays(const SceneDev& s, int32_t li)
 {
-    return s.solid != nullptr && s.culls != 0 && (max(s.H, s.W) >> li) <= kCullPixels;
+    return cull_level(s, li) && s.culls != 0;
 }
 
 // Cameras c0 .. c0 + n - 1 (n <= 64) that some lane of the wavefront (all in one scene) cannot skip; with G
@@ -1333,15 +1340,18 @@ lattice_world(const SceneDev& s, uint32_t px, uint32_t py, uint32_t pz, int32_t 
     }
 }
 
-// All cameras in index order for one parent; returns the occupancy mask.
-template <bool PARTIAL, bool GL, bool UNIFORM>
+// All cameras in index order for one parent; returns the occupancy mask.  CULL: cameras may be left out.  A launch in
+// which no scene can leave out any (carve_culls) runs a copy without that code, here and in the split kernels
+// (64 mixed scenes, us with and without it where it never applies: 100 635 parents, 4 lanes, 460 and 422; 455 118, 2
+// lanes, 760 and 688).
+template <bool PARTIAL, bool GL, bool UNIFORM, bool CULL>
 __device__ uint32_t
 classify_parent(const SceneDev& s, uint32_t px, uint32_t py, uint32_t pz, int32_t li, bool last, uint32_t& tests)
 {
     float wx[3], wy[3], wz[3];
     lattice_world(s, px, py, pz, li, wx, wy, wz);
     uint32_t alive = 0xffu, refine = 0u, inside_any = 0u;
-    if constexpr (UNIFORM)
+    if constexpr (UNIFORM && CULL)
     {
         // the cameras that some lane needs, in index order; a skipped camera counts as a test of every live child
         const float half = 0.5f * s.length * __builtin_ldexpf(1.0f, -li);
@@ -1384,32 +1394,33 @@ classify_parent(const SceneDev& s, uint32_t px, uint32_t py, uint32_t pz, int32_
     return occ;
 }
 
-template <bool PARTIAL, bool GL, bool UNIFORM>
+template <bool PARTIAL, bool GL, bool UNIFORM, bool CULL>
 __device__ __forceinline__ uint32_t
 classify_entry(const SceneDev& s, uint64_t key, int32_t step, uint32_t& tests)
 {
     const int32_t li = step - s.start; // the scene's own octree level
     if (li >= s.level)
         return 0u;
-    return classify_parent<PARTIAL, GL, UNIFORM>(s, key_x(key), key_y(key), key_z(key), li, li == s.level - 1,
-                                                 tests);
+    return classify_parent<PARTIAL, GL, UNIFORM, CULL>(s, key_x(key), key_y(key), key_z(key), li, li == s.level - 1,
+                                                       tests);
 }
 
 // UNIFORM = true for a descriptor shared by the whole wave.  The flag changes
 // no arithmetic; it keeps the wave-uniform and the per-lane instantiations
 // apart, so that the compiler cannot merge the two calls into one per-lane copy.
-template <bool UNIFORM>
+template <bool UNIFORM, bool CULL>
 __device__ __forceinline__ uint32_t
 classify_scene(const SceneDev& s, uint64_t key, int32_t level_i, uint32_t& tests)
 {
     if (s.partial)
-        return s.opengl ? classify_entry<true, true, UNIFORM>(s, key, level_i, tests)
-                        : classify_entry<true, false, UNIFORM>(s, key, level_i, tests);
-    return s.opengl ? classify_entry<false, true, UNIFORM>(s, key, level_i, tests)
-                    : classify_entry<false, false, UNIFORM>(s, key, level_i, tests);
+        return s.opengl ? classify_entry<true, true, UNIFORM, CULL>(s, key, level_i, tests)
+                        : classify_entry<true, false, UNIFORM, CULL>(s, key, level_i, tests);
+    return s.opengl ? classify_entry<false, true, UNIFORM, CULL>(s, key, level_i, tests)
+                    : classify_entry<false, false, UNIFORM, CULL>(s, key, level_i, tests);
 }
 
 // Classification of the kCarveThreads parents of logical block lb (all threads of the block call it).
+template <bool CULL>
 __device__ __forceinline__ void
 classify_block(const uint64_t* __restrict__ parents,
                uint32_t n,
@@ -1429,9 +1440,9 @@ classify_block(const uint64_t* __restrict__ parents,
         const uint32_t sid = key_scene(key);
         const uint32_t s0 = __builtin_amdgcn_readfirstlane(sid);
         if (__all(sid == s0)) // the whole wave carves one scene: camera data and integral bases are scalar
-            mask = classify_scene<true>(wave_uniform(scenes[s0]), key, step, tests);
+            mask = classify_scene<true, CULL>(wave_uniform(scenes[s0]), key, step, tests);
         else
-            mask = classify_scene<false>(scenes[sid], key, step, tests);
+            mask = classify_scene<false, false>(scenes[sid], key, step, tests);
         child_mask[t] = uint8_t(mask);
     }
     uint32_t total;
@@ -1444,6 +1455,7 @@ classify_block(const uint64_t* __restrict__ parents,
         atomicAdd(tests_out, (unsigned long long)tsum);
 }
 
+template <bool CULL>
 __global__ __launch_bounds__(kCarveThreads) void
 carve_classify_kernel(const uint64_t* __restrict__ parents,
                       uint32_t n,
@@ -1455,7 +1467,7 @@ carve_classify_kernel(const uint64_t* __restrict__ parents,
 {
     __shared__ uint32_t lds[kCarveThreads / 64];
     const uint32_t lb = xcd_block(blockIdx.x, gridDim.x); // neighbouring parents read neighbouring pixels
-    classify_block(parents, n, level_i, scenes, child_mask, block_counts, tests_out, lb, lds);
+    classify_block<CULL>(parents, n, level_i, scenes, child_mask, block_counts, tests_out, lb, lds);
 }
 
 // Device-driven form of carve_classify_kernel for a level whose size only the device knows
@@ -1464,6 +1476,7 @@ carve_classify_kernel(const uint64_t* __restrict__ parents,
 // workgroup w runs on XCD w % 8 and takes that XCD's blocks, runs of 16 consecutive blocks whose run
 // index is w % 8 modulo 8 -- the order xcd_block gives a launch-per-level grid -- so neighbouring
 // parents still share an L2, and the workgroups of an XCD balance its blocks among themselves.
+template <bool CULL>
 __global__ __launch_bounds__(kCarveThreads, 4) void
 carve_classify_queue_kernel(const uint64_t* __restrict__ parents,
                             const unsigned long long* __restrict__ dev_n,
@@ -1490,7 +1503,7 @@ carve_classify_queue_kernel(const uint64_t* __restrict__ parents,
         const uint64_t lb = (uint64_t(k / 16u) * 8u + xcd) * 16u + (k % 16u); // increases with k
         if (lb >= nblocks)
             break;
-        classify_block(parents, n, step, scenes, child_mask, block_counts, tests_out, uint32_t(lb), lds);
+        classify_block<CULL>(parents, n, step, scenes, child_mask, block_counts, tests_out, uint32_t(lb), lds);
     }
 }
 
@@ -1500,7 +1513,7 @@ carve_classify_queue_kernel(const uint64_t* __restrict__ parents,
 // child is empty if any camera says so, so the lanes combine exactly by
 // OR / min across the group.  The canonical early-exit count is rebuilt from
 // the first camera that found each child empty.
-template <int G, bool PARTIAL, bool GL, bool UNIFORM>
+template <int G, bool PARTIAL, bool GL, bool CULL>
 __device__ __forceinline__ void
 classify_split(const SceneDev& s, uint64_t key, int32_t level_i, int32_t j, uint32_t& refine, uint32_t& inside,
                uint32_t (&first_empty)[8])
@@ -1514,12 +1527,10 @@ classify_split(const SceneDev& s, uint64_t key, int32_t level_i, int32_t j, uint
     // every camera before it, so the smallest camera of that round that emptied it is its first.
     // All lanes of a group have the same parent, so they run the same rounds.
     uint32_t alive = 0xffu;
-    // With several rounds of cameras, those that no parent of the wavefront needs are left out first: the lanes of
-    // a group test the cameras in turn, the groups' answers are ORed into one mask per 64 cameras, and its cameras
-    // go to the lanes in rounds.  Groups of 16 and 64 lanes have few rounds to save, and small levels pay for the
-    // longer code (a level-7 hull of 8 cameras: 446 instead of 403 us).
-    constexpr bool kCull = UNIFORM && G <= 4;
-    const bool cull = kCull && s.B >= 4 * G && cull_pays(s, level_i);
+    // CULL, with several rounds of cameras: those that no parent of the wavefront needs are left out first.  The
+    // lanes of a group test the cameras in turn, the groups' answers are ORed into one mask per 64 cameras, and its
+    // cameras go to the lanes in rounds.  (Groups of 16 and 64 lanes have few rounds to save.)
+    const bool cull = CULL && s.B >= 4 * G && cull_pays(s, level_i);
     const float half = 0.5f * s.length * __builtin_ldexpf(1.0f, -level_i);
     uint64_t need = 0;
     int32_t c0 = 0, b0 = 0; // first camera of the mask; next camera to look at
@@ -1532,7 +1543,7 @@ classify_split(const SceneDev& s, uint64_t key, int32_t level_i, int32_t j, uint
             {
                 c0 = b0;
                 const int32_t n = min(s.B - c0, 64);
-                if constexpr (kCull)
+                if constexpr (CULL)
                     need = carve_needed<GL, G>(s, c0, n, j, half, wx[1], wy[1], wz[1]);
                 if (PARTIAL && int32_t(__popcll(need)) < n)
                     inside = 0xffu; // a skipped camera sees all children fully inside
@@ -1557,7 +1568,7 @@ classify_split(const SceneDev& s, uint64_t key, int32_t level_i, int32_t j, uint
             b0 += G;
         }
         uint32_t dead = 0u;
-        if (b < s.B && alive != 0u)
+        if (b < s.B && (!CULL || alive != 0u))
             dead = parent_camera<PARTIAL, GL>(s, wx, wy, wz, b, alive, last, refine, inside);
 #pragma unroll
         for (int c = 0; c < 8; ++c)
@@ -1567,14 +1578,14 @@ classify_split(const SceneDev& s, uint64_t key, int32_t level_i, int32_t j, uint
 #pragma unroll
         for (int off = G / 2; off >= 1; off >>= 1)
             alive &= uint32_t(__shfl_xor(int(alive), off, G));
-        if (UNIFORM ? __all(alive == 0u) : alive == 0u)
+        if (CULL ? __all(alive == 0u) : alive == 0u)
             break;
     }
 }
 
 // Scene flags and the classification of one parent by lane j of its group;
 // UNIFORM as for classify_scene.
-template <int G, bool UNIFORM>
+template <int G, bool UNIFORM, bool CULL>
 __device__ __forceinline__ void
 split_scene(const SceneDev& s, uint64_t key, int32_t step, int32_t j, int32_t& B, bool& partial, bool& last,
             bool& active, uint32_t& refine, uint32_t& inside, uint32_t (&first_empty)[8])
@@ -1589,20 +1600,20 @@ split_scene(const SceneDev& s, uint64_t key, int32_t step, int32_t j, int32_t& B
     if (partial)
     {
         if (s.opengl)
-            classify_split<G, true, true, UNIFORM>(s, key, level_i, j, refine, inside, first_empty);
+            classify_split<G, true, true, UNIFORM && CULL>(s, key, level_i, j, refine, inside, first_empty);
         else
-            classify_split<G, true, false, UNIFORM>(s, key, level_i, j, refine, inside, first_empty);
+            classify_split<G, true, false, UNIFORM && CULL>(s, key, level_i, j, refine, inside, first_empty);
     }
     else
     {
         if (s.opengl)
-            classify_split<G, false, true, UNIFORM>(s, key, level_i, j, refine, inside, first_empty);
+            classify_split<G, false, true, UNIFORM && CULL>(s, key, level_i, j, refine, inside, first_empty);
         else
-            classify_split<G, false, false, UNIFORM>(s, key, level_i, j, refine, inside, first_empty);
+            classify_split<G, false, false, UNIFORM && CULL>(s, key, level_i, j, refine, inside, first_empty);
     }
 }
 
-template <int G>
+template <int G, bool CULL>
 __global__ __launch_bounds__(256) void
 carve_classify_split_kernel(const uint64_t* __restrict__ parents,
                             uint32_t n,
@@ -1631,11 +1642,11 @@ carve_classify_split_kernel(const uint64_t* __restrict__ parents,
         const uint32_t sid = key_scene(key);
         const uint32_t s0 = __builtin_amdgcn_readfirstlane(sid);
         if (__all(sid == s0))
-            split_scene<G, true>(wave_uniform(scenes[s0]), key, level_i, j, B, partial, last, active, refine, inside,
-                                 first_empty);
+            split_scene<G, true, CULL>(wave_uniform(scenes[s0]), key, level_i, j, B, partial, last, active, refine,
+                                       inside, first_empty);
         else
-            split_scene<G, false>(scenes[sid], key, level_i, j, B, partial, last, active, refine, inside,
-                                  first_empty);
+            split_scene<G, false, false>(scenes[sid], key, level_i, j, B, partial, last, active, refine, inside,
+                                         first_empty);
     }
 #pragma unroll
     for (int off = G / 2; off >= 1; off >>= 1)
@@ -1992,6 +2003,15 @@ child_lanes(uint32_t n, int32_t max_cameras)
     return uint64_t(n) * uint64_t(G) / 8u <= kChildWaves ? G : 0;
 }
 
+bool
+carve_culls(const SceneDev* scenes, size_t n, int32_t step)
+{
+    return std::any_of(scenes, scenes + n, [&](const SceneDev& s) {
+        const int32_t li = step - s.start;
+        return li < s.level && cull_level(s, li);
+    });
+}
+
 int32_t
 launch_carve_classify(const uint64_t* parents,
                       uint32_t n,
@@ -2002,6 +2022,7 @@ launch_carve_classify(const uint64_t* parents,
                       unsigned long long* tests,
                       const CarveTuning& tune,
                       int32_t max_cameras,
+                      bool culls,
                       hipStream_t st,
                       const unsigned long long* dev_n,
                       int32_t split_hint,
@@ -2019,61 +2040,44 @@ launch_carve_classify(const uint64_t* parents,
     if (split == 16 && max_cameras <= 4)
         split = 4;
     const uint64_t nb = blocks_for(n, kCarveThreads);
-    const auto count = [&] {
-        if (counts)
-            carve_count_kernel<<<nb, kCarveThreads, 0, st>>>(child_mask, n, block_counts, dev_n);
-    };
     if (dev_n != nullptr && split == 1)
     {
         // persistent workgroups: as many as the CUs hold at the kernel's occupancy (3 per CU), a multiple
         // of 8 so that every XCD's queue is served
         const uint64_t grid = std::max<uint64_t>(8, std::min<uint64_t>(768, (nb + 7) / 8 * 8));
-        carve_classify_queue_kernel<<<unsigned(grid), kCarveThreads, 0, st>>>(parents, dev_n, n, level_i, scenes,
-                                                                              child_mask, block_counts, tests, cursors);
+        const auto kernel = culls ? carve_classify_queue_kernel<true> : carve_classify_queue_kernel<false>;
+        kernel<<<unsigned(grid), kCarveThreads, 0, st>>>(parents, dev_n, n, level_i, scenes, child_mask, block_counts,
+                                                         tests, cursors);
+        THULL_LAUNCH_CHECK();
+        return split;
+    }
+    if (split == 1)
+    {
+        const auto kernel = culls ? carve_classify_kernel<true> : carve_classify_kernel<false>;
+        kernel<<<nb, kCarveThreads, 0, st>>>(parents, n, level_i, scenes, child_mask, block_counts, tests);
         THULL_LAUNCH_CHECK();
         return split;
     }
     if (G > 0)
-    {
         carve_classify_child_kernel<<<blocks_for(n, 64 / G), kChildThreads, 0, st>>>(parents, n, level_i, scenes, G,
                                                                                      child_mask, tests, dev_n);
-        THULL_LAUNCH_CHECK();
-        count();
-    }
-    else if (split == 64)
-    {
-        carve_classify_split_kernel<64><<<blocks_for(int64_t(n) * 64, 256), 256, 0, st>>>(parents, n, level_i, scenes,
-                                                                                          child_mask, tests, dev_n);
-        THULL_LAUNCH_CHECK();
-        count();
-    }
-    else if (split == 16)
-    {
-        carve_classify_split_kernel<16><<<blocks_for(int64_t(n) * 16, 256), 256, 0, st>>>(parents, n, level_i, scenes,
-                                                                                          child_mask, tests, dev_n);
-        THULL_LAUNCH_CHECK();
-        count();
-    }
-    else if (split == 4)
-    {
-        carve_classify_split_kernel<4><<<blocks_for(int64_t(n) * 4, 256), 256, 0, st>>>(parents, n, level_i, scenes,
-                                                                                        child_mask, tests, dev_n);
-        THULL_LAUNCH_CHECK();
-        count();
-    }
-    else if (split == 2)
-    {
-        carve_classify_split_kernel<2><<<blocks_for(int64_t(n) * 2, 256), 256, 0, st>>>(parents, n, level_i, scenes,
-                                                                                        child_mask, tests, dev_n);
-        THULL_LAUNCH_CHECK();
-        count();
-    }
     else
     {
-        carve_classify_kernel<<<nb, kCarveThreads, 0, st>>>(parents, n, level_i, scenes, child_mask, block_counts,
-                                                            tests);
+        const auto kernel = split == 64  ? carve_classify_split_kernel<64, false>
+                            : split == 16 ? carve_classify_split_kernel<16, false>
+                            : split == 4  ? (culls ? carve_classify_split_kernel<4, true>
+                                                   : carve_classify_split_kernel<4, false>)
+                                          : (culls ? carve_classify_split_kernel<2, true>
+                                                   : carve_classify_split_kernel<2, false>);
+        kernel<<<blocks_for(int64_t(n) * split, 256), 256, 0, st>>>(parents, n, level_i, scenes, child_mask, tests,
+                                                                    dev_n);
     }
     THULL_LAUNCH_CHECK();
+    if (counts)
+    {
+        carve_count_kernel<<<nb, kCarveThreads, 0, st>>>(child_mask, n, block_counts, dev_n);
+        THULL_LAUNCH_CHECK();
+    }
     return split;
 }
 
