@@ -1355,7 +1355,7 @@ classify_parent(const SceneDev& s, uint32_t px, uint32_t py, uint32_t pz, int32_
     {
         // the cameras that some lane needs, in index order; a skipped camera counts as a test of every live child
         const float half = 0.5f * s.length * __builtin_ldexpf(1.0f, -li);
-        for (int32_t c0 = 0; c0 < s.B; c0 += 64)
+        for (int32_t c0 = 0; c0 < s.B && !__all(alive == 0u); c0 += 64)
         {
             const int32_t n = min(s.B - c0, 64);
             uint64_t need = n < 64 ? (uint64_t(1) << n) - 1u : ~uint64_t(0);
