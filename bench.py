@@ -106,7 +106,7 @@ def carve_profile(run_fn, reps: int = 5) -> dict:
         # algorithmic bytes of carving step i: parents read (4 B), 4 integral reads of 4 B per camera
         # test (early exit), children written (4 B)
         b = 4 * par[i] + 16 * tests[i] + 4 * nxt[i]
-        kernel = {1: "carve_classify_kernel", 0: "carve_classify_queue_kernel"}.get(
+        kernel = {1: "carve_classify_kernel", 0: "carve_classify_queue_kernel", 8: "carve_classify_child_kernel"}.get(
             split[i], f"carve_classify_split_kernel<{split[i]}>")
         levels.append(dict(step=i, level=i + 1, kernel=kernel, ms=float(ms_med[i]), parents=int(par[i]),
                            camera_tests=int(tests[i]), children=int(nxt[i]), bytes=int(b)))

@@ -57,7 +57,9 @@ int thull_ctx_trim(thull_ctx* ctx);
  * (its carving launches one thread per node): max_parents holds 4 values; a level of
  * at most max_parents[0] parents splits each parent's cameras over 64 lanes, up to
  * max_parents[1] over 16, up to max_parents[2] over 4, up to max_parents[3] over 2,
- * larger levels use one lane per parent.  Values are non-decreasing; the results do
+ * larger levels use one lane per parent.  Of the levels with 64 lanes the smallest take a lane
+ * per parent, child and camera instead, and lanes that the scenes' cameras would leave idle are
+ * not used (16 lanes for at most 16 cameras, 4 for at most 4).  Values are non-decreasing; the results do
  * not depend on them.  torchhull_amd.tuning measures and stores the fastest values
  * for a device. */
 int thull_ctx_set_carve_tuning(thull_ctx* ctx, const uint32_t* max_parents);
@@ -176,9 +178,10 @@ int thull_visual_hull_stats(thull_ctx* ctx, int32_t max_levels, int64_t* camera_
 int thull_profile_enable(thull_ctx* ctx, int32_t enabled);
 /* Per carving step i of the last run: classification kernel time (ms, 0 when
  * profiling is off), parent cells, camera tests, resulting child cells and the
- * kernel used (split = 1: one thread per parent; 2/4/16/64: lanes per parent; 0: one thread per parent
- * in the persistent work-queue kernel of a replayed carving loop, whose launches a profiled replay runs
- * eagerly, each timed). */
+ * kernel used (split = 1: one thread per parent; 2/4/16/64: lanes per parent; 8: a lane per parent,
+ * child and camera, the kernel of the smallest levels; 0: one thread per parent in the persistent
+ * work-queue kernel of a replayed carving loop, whose launches a profiled replay runs eagerly, each
+ * timed). */
 int thull_profile_carve(thull_ctx* ctx, int32_t max_levels, float* ms, int64_t* parents, int64_t* tests,
                         int64_t* next, int32_t* split);
 

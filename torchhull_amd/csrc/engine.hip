@@ -374,7 +374,7 @@ struct CarvePlan
     std::vector<int64_t> sig;   // batch shape: scene count and per scene B, H, W, level, flags
     int32_t steps = 0;          // carving steps of the loop
     std::vector<uint32_t> cap;  // list capacities of levels 0 .. steps
-    std::vector<int32_t> split; // lanes per parent of every step
+    std::vector<int32_t> split; // kernel of every step (launch_carve_classify)
     std::vector<uint64_t> roots;
     char* arena = nullptr;
     SceneDev* scenes = nullptr;
@@ -751,7 +751,7 @@ max_cameras(const std::vector<SceneDev>& sd)
 // With `timed`, the launches run eagerly with HIP events around every classification (the profile of
 // a replayed loop: the same kernels as the graph, timed one by one).
 static void
-record_plan(Context& ctx, const CarvePlan& p, const std::vector<SceneDev>& sd, int32_t n, hipStream_t st,
+record_plan(Context& ctx, CarvePlan& p, const std::vector<SceneDev>& sd, int32_t n, hipStream_t st,
             bool timed = false)
 {
     const int32_t steps = p.steps;
@@ -769,9 +769,9 @@ record_plan(Context& ctx, const CarvePlan& p, const std::vector<SceneDev>& sd, i
         const uint32_t nb = blocks_for(p.cap[i], kCarveThreads);
         if (timed)
             THULL_HIP(hipEventRecord(ctx.event(2 * i), st));
-        launch_carve_classify(p.lists[i], p.cap[i], i, p.scenes, p.masks[i], p.bcount[i], tests + i, ctx.tuning,
-                              max_cameras(sd), carve_culls(sd.data(), sd.size(), i), st, counts + i, p.split[i],
-                              p.cursors + 8 * i);
+        p.split[i] = launch_carve_classify(p.lists[i], p.cap[i], i, p.scenes, p.masks[i], p.bcount[i], tests + i,
+                                           ctx.tuning, max_cameras(sd), carve_culls(sd.data(), sd.size(), i), st,
+                                           counts + i, p.split[i], p.cursors + 8 * i);
         if (timed)
             THULL_HIP(hipEventRecord(ctx.event(2 * i + 1), st));
         // the next level's size, clamped to its list's capacity (overflow: the run is repeated)

@@ -49,10 +49,13 @@ constexpr int kCarveThreads = 256;
 // Classifies the 8 children of each parent; writes an 8-bit occupancy mask per
 // parent and the number of occupied children per block of kCarveThreads
 // parents.  `tests` accumulates the number of camera tests (early exit).
-// Returns the number of lanes that share one parent's cameras (1: one thread
-// per parent, carve_classify_kernel; 2/4/16/64: carve_classify_split_kernel<G>).
-// Lanes per parent by level size: G = 64 for at most max_parents[0] parents,
-// 16 up to max_parents[1], 4 up to max_parents[2], else 1.
+// Returns the kernel that ran: the number of lanes that share one parent's cameras (1: one thread
+// per parent, carve_classify_kernel; 2/4/16/64: carve_classify_split_kernel<G>) or kChildSplit.
+// Lanes per parent by level size: G = 64 for at most max_parents[0] parents, 16 up to max_parents[1],
+// 4 up to max_parents[2], 2 up to max_parents[3], else 1.  Of the levels with 64, the smallest take a
+// lane per parent, child and camera, and lanes that the launch's cameras would leave idle are not
+// launched: 16 for at most 16 cameras, 4 for at most 4.
+constexpr int32_t kChildSplit = 8; // carve_classify_child_kernel
 struct CarveTuning
 {
     uint32_t max_parents[4] = { 16384u, 131072u, 1048576u, 1048576u }; // G = 64, 16, 4, 2 up to these sizes

@@ -2032,6 +2032,8 @@ launch_carve_classify(const uint64_t* parents,
     if (n == 0)
         return 0;
     int32_t split = dev_n != nullptr ? split_hint : carve_split_factor(n, tune);
+    if (split == kChildSplit)
+        split = 64; // a plan's hint, from the level that its capacity rounds up
     const int32_t G = split == 64 ? child_lanes(n, max_cameras) : 0;
     // fewer lanes when they still hold a parent's cameras in one round: the others would idle (8197 parents of 8
     // cameras: 64 lanes 38 us, 16 15; 7421 of 10: 38, 21)
@@ -2078,7 +2080,7 @@ launch_carve_classify(const uint64_t* parents,
         carve_count_kernel<<<nb, kCarveThreads, 0, st>>>(child_mask, n, block_counts, dev_n);
         THULL_LAUNCH_CHECK();
     }
-    return split;
+    return G > 0 ? kChildSplit : split;
 }
 
 int32_t
