@@ -2196,7 +2196,7 @@ thull_integral_image_noalloc(thull_ctx* ctx, const void* masks, int32_t dtype, i
         THULL_CHECK(carry_bytes <= kScratchBytes - kScratchJobBytes,
                     "integral_image_noalloc: B * (ceil(H / 32) - 1) * W floats of column carries exceed the 32 MiB "
                     "device scratch (use thull_integral_image)");
-        static_assert(kScratchJobBytes >= 128, "one integral job descriptor fits the job area");
+        static_assert(kScratchJobBytes >= kIntegralJobBytes, "one integral job descriptor fits the job area");
         hipStream_t st = static_cast<hipStream_t>(stream);
         THULL_HIP(hipSetDevice(ctx->c.device));
         char* base = static_cast<char*>(ctx->c.scratch);

@@ -11,6 +11,7 @@ namespace thull
 // torch::cumsum(.., 1, f32) followed by cumsum(.., 2, f32) on CUDA.
 // `job_buf` is device scratch of integral_job_bytes(number of tensors) bytes;
 // `carry` holds integral_carry_floats(B, H, W) floats per tensor.
+constexpr size_t kIntegralJobBytes = 128; // integral_job_bytes(1) at most
 size_t integral_job_bytes(size_t njobs);
 uint64_t integral_carry_floats(int64_t B, int64_t H, int64_t W);
 void launch_integral_image(const void* masks, int32_t dtype, int64_t B, int64_t H, int64_t W, float* out, float* carry,

@@ -91,6 +91,7 @@ struct IntegralJob
     int32_t tile_rows;    // H / kSolidTile
     int32_t tile_pitch;   // ceil(W / 64)
 };
+static_assert(sizeof(IntegralJob) <= kIntegralJobBytes, "callers with a fixed job area reserve kIntegralJobBytes");
 
 __device__ __forceinline__ int32_t
 find_job(const IntegralJob* jobs, int32_t n, uint64_t blk, int pass)
