@@ -3370,8 +3370,9 @@ field_value(const SceneDev& s, uint32_t x, uint32_t y, uint32_t z, Cameras cams)
 // One thread per vertex in numbering order (packed keys).  The gathers of a wave are bound by the
 // vector-memory path (distinct mask lines per instruction); ordering a wave's vertices in 4 x 4 x 4
 // tiles would cut those lines by about 40 %, but whole tiles are too uneven a unit of work (up to
-// 2048 vertices) for a persistent walk, so the kernel keeps the numbering order.
-__global__ __launch_bounds__(256) void
+// 2048 vertices) for a persistent walk, so the kernel keeps the numbering order.  Six waves per SIMD: 80
+// VGPRs, which the compiler passed by 2 when the loop over the cameras was written otherwise.
+__global__ __launch_bounds__(256, 6) void
 field_kernel(const uint64_t* __restrict__ vertices, uint32_t n, const SceneDev* __restrict__ scenes,
              float* __restrict__ values)
 {
