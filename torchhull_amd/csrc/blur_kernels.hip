@@ -676,7 +676,9 @@ blur_tile_kernel(const BlurJob* __restrict__ jobs,
     }
     // Other sizes: the same with the taps of a column taken kTaps at a time, so that a tile value read once
     // still serves up to kTaps pixels of the thread (10 dense 1080p images, k = 11: 0.50 ms with one tile read
-    // and one weight read per tap and pixel, 0.14 ms so, 0.097 ms with the taps compiled in).
+    // and one weight read per tap and pixel, 0.14 ms so, 0.097 ms with the taps compiled in; float64 and float16
+    // outputs, which take this loop for every size: k = 5 0.20 -> 0.12 and 0.22 -> 0.09, k = 11 0.69 -> 0.27 and
+    // 0.59 -> 0.19, sparse k = 3 0.102 -> 0.096 and 0.091).
     constexpr int kTaps = 8;
     To acc[P];
 #pragma unroll
@@ -709,16 +711,17 @@ blur_tile_kernel(const BlurJob* __restrict__ jobs,
             }
         }
     }
+    // (no early exit: with one, this loop stays a loop for __half, and acc an array in private memory: dense k = 3
+    // 85 us instead of 75)
 #pragma unroll
     for (int q = 0; q < P; ++q)
-    {
-        if (q >= nq)
-            break;
-        const int32_t ly = ly0 * P + q;
-        const To result = (band & (1u << q)) ? (sparse ? OutOps<To>::div(acc[q], norm) : acc[q])
-                                             : tile[(ly + h) * LW + lx + h];
-        st(O, int64_t(y0 + ly) * W + x, result);
-    }
+        if (q < nq)
+        {
+            const int32_t ly = ly0 * P + q;
+            const To result = (band & (1u << q)) ? (sparse ? OutOps<To>::div(acc[q], norm) : acc[q])
+                                                 : tile[(ly + h) * LW + lx + h];
+            st(O, int64_t(y0 + ly) * W + x, result);
+        }
 }
 
 // Edge-tile flags and negative-zero flags of B images with a TH x TW tile grid, in whole 32-bit
