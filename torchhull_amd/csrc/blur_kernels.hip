@@ -711,17 +711,24 @@ blur_tile_kernel(const BlurJob* __restrict__ jobs,
             }
         }
     }
-    // (no early exit: with one, this loop stays a loop for __half, and acc an array in private memory: dense k = 3
-    // 85 us instead of 75)
+    // With an early exit this loop stays a loop for __half, and acc an array in private memory (dense k = 3 85 us
+    // instead of 75); float64 is 2 % faster with it (dense k = 11 303 us and 310).
+    constexpr bool kExit = !std::is_same_v<To, __half>;
 #pragma unroll
     for (int q = 0; q < P; ++q)
-        if (q < nq)
+    {
+        if (q >= nq)
         {
-            const int32_t ly = ly0 * P + q;
-            const To result = (band & (1u << q)) ? (sparse ? OutOps<To>::div(acc[q], norm) : acc[q])
-                                                 : tile[(ly + h) * LW + lx + h];
-            st(O, int64_t(y0 + ly) * W + x, result);
+            if constexpr (kExit)
+                break;
+            else
+                continue;
         }
+        const int32_t ly = ly0 * P + q;
+        const To result = (band & (1u << q)) ? (sparse ? OutOps<To>::div(acc[q], norm) : acc[q])
+                                             : tile[(ly + h) * LW + lx + h];
+        st(O, int64_t(y0 + ly) * W + x, result);
+    }
 }
 
 // Edge-tile flags and negative-zero flags of B images with a TH x TW tile grid, in whole 32-bit
