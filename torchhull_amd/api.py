@@ -183,7 +183,7 @@ class _Run:
         _lib.check(_lib.lib().thull_visual_hull_fetch_field(self.ctx, i, _ptr(idx), _ptr(vals), self.stream))
         r = (1 << level) + 1
         # to_sparse_coo_tensor (visual_hull_cuda.cu:575-577); indices are sorted and unique, so coalescing would
-        # only sort them again (a level-8 field: 180 of 732 us) and add every value to zero, as here
+        # only sort them again (a level-8 field: 266 of 732 us) and add every value to zero, as here
         return torch.sparse_coo_tensor(idx, vals.add_(0.0), (1, r, r, r), is_coalesced=True)
 
     def candidates(self) -> list[torch.Tensor]:

@@ -788,7 +788,7 @@ run_blur_rb(std::vector<BlurJob>& jobs, BlurJob* djobs, Uploader& up, int k, boo
     }
     const int32_t n = int32_t(jobs.size());
     // the tile pass has its own block layout: a second table behind the first, and one copy for both (a copy
-    // between the passes kept 30 1080p images waiting: 162 -> 157 us)
+    // between the passes kept 30 1080p images waiting: 162 -> 160 us, nothing on images seen for the first time)
     jobs.resize(2 * size_t(n));
     for (int32_t i = 0; i < n; ++i)
     {
