@@ -31,6 +31,21 @@ def test_choice_is_the_best_of_all_cuts(seed):
     assert chosen == sorted(chosen)
 
 
+def test_present_thresholds_stay_where_they_cost_next_to_nothing():
+    sizes = [1000, 30000, 300000, 3000000]
+    fast = dict(zip(sizes, (64, 16, 4, 1)))
+    samples = {g: [(n, 1.0 if g == fast[n] else 2.0) for n in sizes] for g in (64, 16, 4, 2, 1)}
+    # the last two cut the same sizes as the choice does, the first ones do not
+    chosen, cost = tuning.choose_thresholds(samples, present=[100, 20000, 310000, 2900000])
+    assert cost == 4.0
+    assert chosen[2:] == [310000, 2900000]
+    assert 1000 <= chosen[0] < 30000 <= chosen[1] < 300000
+    # a level that hardly counts may go to the present threshold's lanes
+    weights = [1.0, 1.0, 1.0, 1e-4]
+    chosen, cost = tuning.choose_thresholds(samples, weights, [1000, 30000, 300000, 3000000])
+    assert chosen == [1000, 30000, 300000, 3000000] and cost == pytest.approx(3.0002)
+
+
 def test_thresholds_lie_between_the_measured_sizes():
     sizes = [1000, 30000, 31000, 900000]
     fast = dict(zip(sizes, (64, 16, 4, 1)))

@@ -11,14 +11,14 @@ levels that ask for 64 lanes the library gives the smallest a kernel of their ow
 and scenes of few cameras fewer lanes (`split_for` with `cameras`).  It then picks
 the four level-size thresholds that minimise the sum of all measured levels, each
 as a share of its workload's whole call, so that a preview counts as much as a
-level-11 hull.  A threshold lies half way (by the logarithm) between the measured
-sizes around it.  The choice never changes a result, only its speed.
+level-11 hull.  Present thresholds stay where they cost next to nothing (SLACK); a
+new one lies half way (by the logarithm) between the measured sizes around it.  The choice never changes a result, only its speed.
 
 `python -m torchhull_amd.tuning --out torchhull_amd/carve_tuning.json` tunes on
 `workloads(seed)`: single hulls of levels 6 to 11 and mixed batches, drawn over the
-range of cameras, image sizes, conventions and blurs; checks the choice on another
-draw of them; and writes the thresholds, which `_lib.context` applies to every new
-context when the file is there.
+range of cameras, image sizes, conventions and blurs, every other batch as a replayed
+loop; checks the choice on another draw of them; and writes the thresholds, which
+`_lib.context` applies to every new context when the file is there.
 """
 
 from __future__ import annotations
@@ -112,10 +112,16 @@ def _between(lo: int, hi: int) -> int:
     return rounded if lo <= rounded < hi else t
 
 
-def choose_thresholds(samples: dict[int, list[tuple[int, float]]],
-                      weights: Sequence[float] | None = None) -> tuple[list[int], float]:
+# A choice between thresholds whose costs differ by less than this is the draw's, not the device's (the own
+# thresholds of another draw gain 0.2 % on it): the present ones stay.
+SLACK = 0.002
+
+
+def choose_thresholds(samples: dict[int, list[tuple[int, float]]], weights: Sequence[float] | None = None,
+                      present: Sequence[int] | None = None) -> tuple[list[int], float]:
     """Thresholds minimising the summed (weighted) level time; samples[G] = [(parents, ms), ...] over the same
-    levels.  G may only fall as levels grow, so the sizes are cut into five runs: a dynamic program over the cuts."""
+    levels.  G may only fall as levels grow, so the sizes are cut into five runs: a dynamic program over the cuts.
+    Of the `present` thresholds, those stay that leave the sum within SLACK of the least, from the last on."""
     levels = [n for n, _ in samples[1]]
     weights = [1.0] * len(levels) if weights is None else weights
     sizes = sorted(set(levels))
@@ -140,7 +146,14 @@ def choose_thresholds(samples: dict[int, list[tuple[int, float]]],
     for cut in reversed(cuts[1:]):
         at = cut[at]
         chosen.append(0 if at == 0 else _MAX if at == len(sizes) else _between(sizes[at - 1], sizes[at]))
-    return chosen[::-1], best[-1]
+    chosen, least = chosen[::-1], best[-1]
+    total = least
+    for q in reversed(range(_N if present is not None else 0)):
+        trial = chosen[:q] + [present[q]] + chosen[q + 1:]
+        cost_trial = _shares(samples, weights, trial)
+        if trial == sorted(trial) and cost_trial <= least * (1.0 + SLACK):
+            chosen, total = trial, cost_trial
+    return chosen, total
 
 
 def _shares(samples: dict[int, list[tuple[int, float]]], weights: Sequence[float], max_parents: Sequence[int]) -> float:
@@ -166,8 +179,11 @@ def measure(runs: Sequence[Callable[[], object]], device_index: int = 0,
                 times.append(1e3 * (time.perf_counter() - t0))
             for g, force in _FORCE.items():
                 set_carve_tuning(ctx, force)
+                _lib.check(_lib.lib().thull_ctx_trim(ctx))
+                run()  # a replayed batch plans its loop with this G
                 samples[g].extend(measure_levels(run, ctx, reps))
             set_carve_tuning(ctx, saved)
+            _lib.check(_lib.lib().thull_ctx_trim(ctx))
             weights += [1.0 / statistics.median(times[2:])] * (len(samples[1]) - len(weights))
     finally:
         set_carve_tuning(ctx, saved)
@@ -180,7 +196,7 @@ def tune_carving(workloads: Sequence[Callable[[], object]], device_index: int = 
     context's present thresholds."""
     saved = get_carve_tuning(_lib.context(device_index))
     samples, weights = measure(workloads, device_index, reps)
-    chosen, _ = choose_thresholds(samples, weights)
+    chosen, _ = choose_thresholds(samples, weights, saved)
     return {"max_parents": chosen, "shares": round(_shares(samples, weights, chosen), 4),
             "default_shares": round(_shares(samples, weights, saved), 4),
             "levels": [{"parents": n, "weight": round(weights[i], 4),
@@ -200,8 +216,9 @@ def load(path: pathlib.Path = DEFAULT_PATH) -> list[int] | None:
     return None
 
 
-def workloads(seed: int, device: torch.device, singles: int = 288) -> Iterator[tuple[str, Callable[[], object]]]:
-    """Single hulls over levels 6 to 11, 4 to 64 cameras and 192 to 2048 pixels, and batches of mixed scenes."""
+def workloads(seed: int, device: torch.device, singles: int = 288,
+              batches: int = 36) -> Iterator[tuple[str, Callable[[], object]]]:
+    """Single hulls over levels 6 to 11, 4 to 64 cameras and 192 to 2048 pixels, and batches of 2 to 64 mixed scenes."""
     from . import api, synthetic
 
     rng = np.random.default_rng(seed)
@@ -226,12 +243,13 @@ def workloads(seed: int, device: torch.device, singles: int = 288) -> Iterator[t
         m = sc.masks if sc.blur is None else api.gaussian_blur(sc.masks, *sc.blur, sparse=True, dtype=torch.float32)
         yield (f"level {level}, {spec.n_cameras} x {spec.resolution}^2{' partial' if partial else ''}",
                lambda a=args(sc, m): api.visual_hull(**a))
-    for n, top in ((4, 8), (10, 9), (24, 9), (64, 9)):
+    for i in range(batches):
+        n, top, graph = log_uniform(2, 64), int(rng.integers(7, 10)), i % 2 == 1
         scenes = synthetic.mixed_scenes(n, seed=int(rng.integers(1 << 30)), device=device, max_level=top)
         blurred = api.gaussian_blur_batch([sc.masks for sc in scenes], *scenes[0].blur, sparse=True,
                                           dtype=torch.float32)
-        yield (f"{n} mixed scenes up to level {top}",
-               lambda b=[args(sc, m) for sc, m in zip(scenes, blurred)]: api.visual_hull_batch(b))
+        yield (f"{n} mixed scenes up to level {top}{', replayed' if graph else ''}",
+               lambda b=[args(sc, m) for sc, m in zip(scenes, blurred)], g=graph: api.visual_hull_batch(b, graph=g))
 
 
 def main() -> None:
