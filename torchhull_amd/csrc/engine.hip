@@ -806,8 +806,9 @@ check_scene(const thull_scene& sc)
 
 // Solid maps and the field by bricks cost a few launches and a sixteenth of a pass over the masks, and save camera
 // tests and samples of the scenes' surface cells, about 4^level of them in every camera: they are used from
-// kMinCellCameras cell-cameras in the scenes a run starts with (16.8 million, 64 cameras at level 9: 1.96 -> 1.60 ms;
-// 6.4 million in 10 mixed scenes: 1.66 -> 1.75; 0.7 million, 10 cameras at level 8: 0.50 -> 0.54).
+// kMinCellCameras cell-cameras in the scenes a run starts with (16.8 million, 64 cameras at level 9: 1.75 -> 1.41 ms;
+// 6.3 million, 24 cameras at level 9: 0.79 -> 0.74, and in 10 mixed scenes: 1.55 -> 1.68; 3.3 million, 50 cameras at
+// level 8: 1.06 -> 1.03; 0.7 million, 10 cameras at level 8: 0.41 -> 0.47).
 static bool
 solid_maps_pay(const thull_scene* scenes, int32_t n)
 {
